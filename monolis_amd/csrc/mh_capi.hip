@@ -1432,12 +1432,8 @@ int monolis_hip_matrix_create_by_simple_mesh(monolis_hip_matrix** out, int n_nod
   int nz = 0;
   MH_TRY(mh::pattern_by_simple_mesh(n_node, n_base, n_elem, elem, index, item, &nz, c->stream));
   // values start at zero, as monolis_alloc_nonzero_pattern_mat_val_R leaves them
-  mh::DevArray<double> zeros;
-  const size_t nv = (size_t)nz * n_dof * n_dof;
-  MH_TRY(zeros.alloc(nv));
-  MH_HIP(hipMemsetAsync(zeros.p, 0, sizeof(double) * (nv ? nv : 1), c->stream));
   Matrix* M = nullptr;
-  MH_TRY(mh::matrix_create(&M, n_node, n_node, nz, n_dof, index.p, item.p, zeros.p, c->stream));
+  MH_TRY(mh::matrix_create_zero(&M, n_node, nz, n_dof, index.p, item.p, false, c->stream));
   auto* H = new monolis_hip_matrix();
   H->M = M;
   *out = H;
@@ -1590,12 +1586,8 @@ int monolis_hip_matrix_create_by_simple_mesh_C(monolis_hip_matrix_C** out, int n
   int nz = 0;
   MH_TRY(mh::pattern_by_simple_mesh(n_node, n_base, n_elem, elem, index, item, &nz, c->stream));
   // values start at zero (monolis_alloc_nonzero_pattern_mat_val_C)
-  mh::DevArray<double> zeros;
-  const size_t nd = (size_t)nz * n_dof * n_dof * 2;
-  MH_TRY(zeros.alloc(nd ? nd : 1));
-  MH_HIP(hipMemsetAsync(zeros.p, 0, sizeof(double) * (nd ? nd : 1), c->stream));
   Matrix* M = nullptr;
-  MH_TRY(mh::matrix_create_complex(&M, n_node, n_node, nz, n_dof, index.p, item.p, zeros.p, c->stream));
+  MH_TRY(mh::matrix_create_zero(&M, n_node, nz, n_dof, index.p, item.p, true, c->stream));
   auto* H = new monolis_hip_matrix_C();
   H->M = M;
   *out = H;

@@ -123,6 +123,7 @@ struct VBlock {
 struct Matrix {
   int n = 0, np = 0, nz = 0, b = 0;
   int nslices = 0;
+  int max_width = 0;                        // longest row
   size_t nslots = 0;
   DevArray<int> slice_ptr, rowptr, col;     // SELL pattern (rowptr = monolis index)
   // 16-bit column deltas (col - row), two slots per 32-bit word (SellView::col16);
@@ -157,6 +158,9 @@ struct Matrix {
 
 int matrix_create(Matrix** out, int n, int np, int nz, int b, const int* index, const int* item,
                   const double* A, hipStream_t s);
+// A square matrix of zeros on a given pattern.
+int matrix_create_zero(Matrix** out, int n, int nz, int b, const int* index, const int* item, bool cplx,
+                       hipStream_t s);
 int matrix_set_values(Matrix* M, const double* A, hipStream_t s);
 // Complex matrix: A holds NZ*b*b complex values, interleaved (re, im) doubles;
 // matrix_set_values refills it from the same layout.
@@ -180,6 +184,9 @@ int vdiag_make_fp32(Matrix& M, hipStream_t s);
 template <typename T>
 int vdiag_apply(const Matrix& M, const T* x, T* y, hipStream_t s);
 int matrix_make_fp32(Matrix* M, hipStream_t s);
+// Stored values in monolis's block CSR order (device pointers).
+int launch_sell_gather(const Matrix& M, const double* val, double* A, hipStream_t s);
+int launch_sell_gather(const Matrix& M, const zd* val, zd* A, hipStream_t s);
 int matrix_transpose(Matrix* M, hipStream_t s);
 
 template <typename TV>

@@ -52,6 +52,40 @@ def test_pattern_matches_oracle(case):
     assert np.array_equal(dm.mat.index, index) and np.array_equal(dm.mat.item, item)
 
 
+def test_pattern_hub_node_takes_the_sorted_pairs():
+    """A node in so many elements that its row has more candidate columns than one wavefront sorts on chip."""
+    n_node = 400
+    rng = np.random.default_rng(8)
+    elems = np.array([[0, *rng.choice(np.arange(1, n_node), 3, replace=False)] for _ in range(300)], np.int32)
+    dm = api.device_matrix_by_simple_mesh(n_node, 1, elems)
+    index, item = oracle.pattern_by_simple_mesh(n_node, elems)
+    assert np.array_equal(dm.mat.index, index) and np.array_equal(dm.mat.item, item)
+
+
+# strips of one, two, four and more 64-value pieces; 16, 8 and 4 rows of LDS per workgroup; rows too
+# long for LDS; an element that lists a node twice
+@pytest.mark.parametrize("n_base, b, n_node, n_elem, dup",
+                         [(1, 1, 5, 9, False), (2, 4, 67, 150, False), (8, 1, 300, 700, False), (4, 5, 200, 500, False),
+                          (10, 6, 90, 130, False), (20, 2, 150, 100, False), (8, 8, 130, 260, False),
+                          (4, 3, 80, 120, True)])
+def test_element_assembly_layouts_bit_identical(n_base, b, n_node, n_elem, dup):
+    rng = np.random.default_rng(n_base * 100 + b)
+    elems = np.array([rng.choice(n_node, n_base, replace=False) for _ in range(n_elem)], np.int32)
+    if dup:
+        elems[17, 3] = elems[17, 1]
+    Ke = element_matrices(n_elem, n_base * b, seed=b, spd=False)
+    dm = api.device_matrix_by_simple_mesh(n_node, b, elems)
+    mo = _oracle_mat(n_node, b, elems)
+    assert np.array_equal(dm.mat.index, mo.index) and np.array_equal(dm.mat.item, mo.item)
+    start = rng.uniform(-1, 1, len(mo.A))
+    dm.set_values(start)
+    assert np.array_equal(dm.values(), start)
+    mo.A[:] = start
+    dm.add_elements(elems, Ke)
+    oracle.add_elements(mo, elems, Ke)
+    assert np.array_equal(dm.values(), mo.A)
+
+
 def test_pattern_rejects_bad_node_ids():
     h = ctypes.c_void_p()
     e = np.array([[0, 5]], np.int32)
