@@ -46,10 +46,16 @@ int context(Context** c);
 // The context if it is already initialised (never initialises: that allocates), else null.
 Context* context_if_ready();
 
+// Device memory of at least `bytes` for work on the library's stream; *cap is
+// handed back to dev_free, which keeps the block for a later allocation.
+int dev_alloc(void** p, size_t bytes, size_t* cap);
+void dev_free(void* p, size_t cap);
+
 template <typename T>
 struct DevArray {
   T* p = nullptr;
   size_t n = 0;
+  size_t cap = 0;  // bytes of the block (0: not from the pool)
   int alloc(size_t count);
   void release();
   ~DevArray() { release(); }
