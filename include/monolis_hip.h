@@ -230,11 +230,13 @@ int monolis_hip_batch_solve(monolis_hip_batch* B, const double* b, double* x, in
 int monolis_hip_batch_num_configs(void);
 int monolis_hip_batch_config(int cfg, int* threads, int* unroll);
 /* Selects configuration cfg for the following solves (the autotuner's choice
- * otherwise; 0 before any tuning). */
+ * otherwise; before any tuning 15, the solver that keeps the vectors on chip,
+ * or 0 for a batch with a system too large for it, where 15 runs 11). */
 int monolis_hip_batch_set_config(monolis_hip_batch* B, int cfg);
 /* Team split of configuration cfg (0: one workgroup per system; s > 0: systems
  * whose estimated work exceeds s/4 of one workgroup's balanced share are solved
- * by a team of up to 32 workgroups) and the number of slots (one per workgroup
+ * by a team of up to 32 workgroups; 1 for configuration 15: as many workgroups
+ * as hold the system on chip) and the number of slots (one per workgroup
  * task) and teams its schedule for B has. */
 int monolis_hip_batch_schedule(monolis_hip_batch* B, int cfg, int* split, int* nslot, int* nteam);
 /* Longest time in seconds (default 5, at most 600) that one team barrier waits

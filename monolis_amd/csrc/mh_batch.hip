@@ -8,7 +8,9 @@
 // monolis_solve_R were called once per system.
 //
 // Layout: a system-aligned SELL-64 -- every system starts on a fresh 64-row
-// slice, so a workgroup walks only its own slices.  Two persistent kernels:
+// slice, so a workgroup walks only its own slices.  Three persistent kernels:
+//  * k_res_cg (mh_resident.hpp): the vectors stay on chip; the default where it
+//    fits;
 //  * k_batch_cg: each workgroup takes systems wg, wg + G, ... (largest first) and
 //    runs the whole CG loop with workgroup barriers only;
 //  * k_batch_sched: the largest systems are split over teams of up to 32
@@ -24,6 +26,7 @@
 
 #include "mh_batch.hpp"
 #include "mh_kernels.hpp"
+#include "mh_resident.hpp"
 
 namespace mh {
 
@@ -65,13 +68,6 @@ struct BatchView {
   const double* val;
   const int* rowlen;        // per SELL row (padding rows: 0)
   const double* dinv;       // diagonal preconditioner per global row (1/a_ii, zero pivot -> 1)
-};
-
-// Per-system results written by the solver kernel.
-struct BatchOut {
-  int* iters;
-  double* resid;
-  int* status;   // 0 converged, 1 not converged, 2 zero rhs, 3 a team wait gave up
 };
 
 // One SELL row times a vector whose entry c is gather(c).
@@ -594,6 +590,14 @@ __global__ void k_batch_fill(int nsys_rows_total, const int* __restrict__ sell_s
     } break;                                         \
   }
 
+// Configuration 15: the on-chip CG (mh_resident.hpp).  512 Poisson systems of
+// 10^3..40^3 rows: 19.0 ms against 51.1 for the best of the others (the
+// vectors' 108 of 190 bytes per row and iteration stay on chip).  It is the
+// default of every batch it fits; one with a system it does not fit runs
+// kCfgFallback instead (also when configuration 15 is asked for).
+constexpr int kCfgResident = 15;
+constexpr int kCfgFallback = 11;
+
 // Team schedule of a configuration (NT threads per workgroup, `resident`
 // workgroups at once, split factor ts): the estimated work of a system is
 // (entries + 6 rows) x rows^(1/3) (the SpMV and vector bytes times an iteration
@@ -657,14 +661,20 @@ int build_sched(const Batch& B, int NT, int resident, int ts, BatchSched& S, hip
 
 }  // namespace
 
-int batch_num_configs() { return 15; }
+int batch_num_configs() { return kCfgResident + 1; }
 
 void batch_config_info(int cfg, int* threads, int* unroll) {
+  if (cfg == kCfgResident) {
+    *threads = kResNT;
+    *unroll = 8;
+    return;
+  }
   MH_BATCH_CFG(cfg, *threads = NT; *unroll = UU);
 }
 
 int batch_config_split(int cfg) {
   int ts = 0;
+  if (cfg == kCfgResident) return 1;
   MH_BATCH_CFG(cfg, ts = TS);
   return ts;
 }
@@ -694,10 +704,22 @@ static int ensure_sched(Batch& B, int cfg, BatchSched** out, hipStream_t s) {
   return 0;
 }
 
+// The configuration that a launch of cfg runs.
+static int effective_config(const Batch& B, int cfg) {
+  return cfg == kCfgResident && !B.res.fits ? kCfgFallback : cfg;
+}
+
 int batch_schedule_info(Batch& B, int cfg, int* split, int* nslot, int* nteam, hipStream_t s) {
   if (cfg < 0 || cfg >= batch_num_configs()) {
     set_error("batch config %d out of range", cfg);
     return -2;
+  }
+  cfg = effective_config(B, cfg);
+  if (cfg == kCfgResident) {
+    *split = 1;
+    *nslot = B.res.nmem;
+    *nteam = B.res.nteam;
+    return 0;
   }
   *split = batch_config_split(cfg);
   *nslot = B.nsys;
@@ -712,6 +734,8 @@ int batch_schedule_info(Batch& B, int cfg, int* split, int* nslot, int* nteam, h
 
 int batch_aborted(Batch& B, int cfg, int* aborted, hipStream_t s) {
   *aborted = 0;
+  cfg = effective_config(B, cfg);
+  if (cfg == kCfgResident) return res_aborted(B.res, aborted, s);
   if (cfg < 0 || cfg >= (int)B.sched.size() || !B.sched[cfg] || batch_config_split(cfg) == 0) return 0;
   // the sticky flag: set by any launch since the last check, then cleared
   int flag = 0;
@@ -825,6 +849,13 @@ int batch_create(Batch** out, int nsys, const int* sys_row_h, int n, int nz, con
   k_batch_fill<<<(total + 255) / 256, 256, 0, s>>>(total, d_sell_sys.p, B->sys_slice.p, B->sys_row.p, d_idx.p, d_item.p,
                                                    d_A.p, B->slice_ptr.p, B->col.p, B->val.p, B->rowlen.p, B->dinv.p);
   MH_HIP(hipGetLastError());
+  std::vector<ResSystem> rs((size_t)nsys);
+  for (int k = 0; k < nsys; ++k)
+    rs[k] = ResSystem{sys_slice[k], B->h_slices[k], sys_row_h[k], B->h_rows[k],
+                      ((double)B->h_nnz[k] + 6.0 * B->h_rows[k]) * std::cbrt(std::max((double)B->h_rows[k], 1.0))};
+  MH_TRY(res_plan_build(B->res, rs, slice_ptr.data(), nslices, B->slice_ptr.p, B->col.p, B->rowlen.p, nullptr,
+                        cu_count_batch(), s));
+  if (B->res.fits) B->cfg = kCfgResident;
   MH_HIP(hipStreamSynchronize(s));
   *out = B.release();
   return 0;
@@ -842,13 +873,18 @@ int batch_solve(Batch& B, const BatchParams& P, const double* b, double* x, int 
     set_error("batch config %d out of range", cfg);
     return -2;
   }
+  cfg = effective_config(B, cfg);
   BatchSched* S = nullptr;
-  if (batch_config_split(cfg) > 0) MH_TRY(ensure_sched(B, cfg, &S, s));
+  if (cfg != kCfgResident && batch_config_split(cfg) > 0) MH_TRY(ensure_sched(B, cfg, &S, s));
   // k_batch_cg: one workgroup per system while they fit two per CU, else
   // grid-stride over systems
   int grid = std::min(B.nsys, cu_count_batch() * 2);
   if (grid < 1) grid = 1;
   auto enqueue = [&]() -> int {
+    if (cfg == kCfgResident) {
+      const ResArgs A{b, x, z, p, O, nullptr, P.max_iter, P.tol, P.init_x, P.precond};
+      return res_launch(B.res, B.slice_ptr.p, B.val.p, B.dinv.p, A, B.nsys, B.wait_s, s);
+    }
     const int nctl = S ? 2 + S->nteam : 0;
     k_batch_reset<<<(std::max(B.nsys, nctl) + 255) / 256, 256, 0, s>>>(B.nsys, B.iters.p, B.resid.p, B.status.p,
                                                                          S ? S->ctl.p : nullptr, nctl);

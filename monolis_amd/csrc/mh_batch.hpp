@@ -5,6 +5,7 @@
 #include <vector>
 
 #include "mh_internal.hpp"
+#include "mh_resident.hpp"
 
 namespace mh {
 
@@ -39,7 +40,8 @@ struct Batch {
   DevArray<double> resid;
   std::vector<int> h_rows, h_nnz, h_slices;  // per system (schedule building)
   std::vector<std::unique_ptr<BatchSched>> sched;  // per configuration, built on first use
-  int cfg = 0;  // tuned launch configuration
+  ResPlan res;  // on-chip solver's members (res.fits: usable)
+  int cfg = 0;  // launch configuration: the on-chip solver where it fits, 0 otherwise, or the tuned one
   double wait_s = 5.0;  // longest team wait before a launch gives up
   // captured launch (replayed while arguments are unchanged)
   hipGraphExec_t graph_exec = nullptr;
@@ -53,7 +55,8 @@ struct Batch {
 int batch_num_configs();
 void batch_config_info(int cfg, int* threads, int* unroll);
 // Team split of a configuration: 0 = one workgroup per system, else systems whose
-// estimated work exceeds split/4 of a workgroup's balanced share get teams.
+// estimated work exceeds split/4 of a workgroup's balanced share get teams (1: the
+// on-chip solver, whose teams follow from what a workgroup can hold).
 int batch_config_split(int cfg);
 int batch_create(Batch** out, int nsys, const int* sys_row_host, int n, int nz, const int* index, const int* item,
                  const double* A, hipStream_t s);

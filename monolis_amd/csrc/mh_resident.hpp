@@ -1,0 +1,457 @@
+// On-chip CG: a scalar system solved by one workgroup, or by a team of them,
+// whose vectors never leave the CUs.
+//
+// A member owns a contiguous range of the system's 64-row slices, at most
+// RP * 8 of them.  p of its rows and of the rows it couples to (its halo) lives
+// in LDS; x, r and q / z live in registers, RP rows per thread.  An iteration
+// then streams only the matrix -- 8 bytes of value and 2 bytes of LDS index per
+// entry -- and the preconditioner's 8 bytes per row: about 80 bytes per row of a
+// 7-point system against 190 with the vectors in memory.  512 Poisson systems of
+// 10^3..40^3 rows: 51.1 -> 19.0 ms, 1.377e9 row-iterations at 72 G/s (5.8 TB/s of
+// those bytes): bound by the matrix stream.
+//
+// Team members exchange two things, through agent-scope stores and loads that
+// bypass the XCD's L2 (no cache write-back or invalidation): the partial sums of
+// the two reductions of an iteration, and z of the rows some other member
+// reads.  Every member updates its copy of a halo row's p as its owner does,
+// p = z + beta p, so p itself is never exchanged.
+#pragma once
+
+#include <memory>
+#include <vector>
+
+#include "mh_internal.hpp"
+#include "mh_kernels.hpp"
+
+namespace mh {
+
+constexpr int kResNT = 512;                 // threads per member: two wavefronts per SIMD, 256 VGPRs each
+constexpr int kResNW = kResNT / kWave;
+constexpr int kResTeamMax = 32;             // workgroups per team at most
+constexpr int kResLds = 20352;              // doubles of LDS for p (159 KB of the CU's 160)
+constexpr int kResSpinMax = 1 << 24;        // polls of one team wait at most (a bound that needs no clock)
+constexpr int kResIterRR = 200;             // residual replacement (CG.f90:91-95)
+constexpr int kResRowsLarge = 26;           // RP: 13,312 rows per member (150 VGPRs of vectors)
+constexpr int kResRowsSmall = 8;            // RP: 4,096 rows, two workgroups per CU
+
+struct ResMember {
+  int sys, rank, T, team;
+  int slice0, nsl;      // own slices
+  int row0, nown;       // first own row (global) and own rows
+  int sysrow0, sysslice0, sysrows;
+  int halo_off, halo_cap, nhalo;
+  int w8;               // no own slice is wider than 8 slots
+  int pad;
+};
+
+struct ResView {
+  int nmem;
+  const ResMember* mem;
+  const int* slice_ptr;   // SELL slot offsets
+  const int* g_ptr;       // per slice: first group of 8 LDS indices
+  const double* val;      // SELL values, one plane per slot
+  const uint4* lcol;      // per group and lane: 8 16-bit LDS indices
+  const unsigned char* expf;  // per slice: some other member reads a row of it
+  const double* dinv;     // diagonal preconditioner per row
+  const int* halo;        // global rows, per member
+  int* ctl;               // [0] next member, [1] abort flag, [2 + t] arrivals of team t
+  double* part;           // per team: 2 alternating sets x kResTeamMax x 2 partial sums
+  long long limit;        // wall-clock ticks one wait may last
+  int* sticky;            // set with the abort flag, cleared only by the host
+};
+
+// Per-system results.
+struct BatchOut {
+  int* iters;
+  double* resid;
+  int* status;   // 0 converged, 1 not converged, 2 zero rhs, 3 a team wait gave up
+};
+
+struct ResArgs {
+  const double* b;
+  double* x;
+  double* z;       // exported z (written for exported slices only)
+  double* p;       // exported p (residual replacement only)
+  BatchOut out;
+  double* hist;    // residual history of the only system, or null
+  int max_iter;
+  double tol;
+  int init_x, precond;
+};
+
+__device__ __forceinline__ void st_agent(double* p, double v) {
+  __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ double ld_agent(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// The value itself, as something the compiler cannot carry over from an earlier
+// use: the per-row addresses and conditions of an unrolled pass are then formed
+// in the pass, instead of being kept for the whole solve (RP of each, which
+// spilled thousands of registers).
+__device__ __forceinline__ int fresh_s(int v) {
+  v = __builtin_amdgcn_readfirstlane(v);
+  asm volatile("" : "+s"(v));
+  return v;
+}
+__device__ __forceinline__ int fresh_v(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+// i * 8 < left as a condition of its own: the compiler would otherwise thread
+// the branches of an unrolled pass (one that fails implies the rest), which
+// multiplies its code and its live registers.
+__device__ __forceinline__ bool res_on(int left, int i) {
+  asm volatile("" : "+s"(left));
+  return i * kResNW < left;
+}
+
+// One member's part of one system.
+template <int RP, bool W8>
+__device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, const ResArgs& a, double* lds, double* red,
+                                       int* flag) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
+  const int own = m.nsl * kWave;  // LDS: own rows (whole slices), halo rows, one zero
+  const int T = m.T;
+  double x[RP], r[RP], q[RP];     // row i of a thread: slice w + i*8 of the member, its lane
+#pragma unroll
+  for (int i = 0; i < RP; ++i) x[i] = r[i] = q[i] = 0.0;
+  // lane i holds the slot and group offsets and the export bit of slice w + i*8
+  int kreg = 0, wreg = 1, greg = 0;
+  bool ereg = false;
+  {
+    const int s = w + lane * kResNW;
+    if (lane < RP && s < m.nsl) {
+      kreg = V.slice_ptr[m.slice0 + s];
+      wreg = V.slice_ptr[m.slice0 + s + 1] - kreg;
+      greg = V.g_ptr[m.slice0 + s];
+      ereg = T > 1 && V.expf[m.slice0 + s] != 0;
+    }
+  }
+  const unsigned long long exports = __ballot(ereg);
+  // A pass over the thread's rows: f(i, l, real, g) with l the row's LDS index,
+  // real whether it is a row of the system, g its global row (lanes past the
+  // system's last row take that row).
+  auto for_rows = [&](auto&& f) {
+    const int left = fresh_s(m.nsl - w), l0 = fresh_v(w * kWave + lane), g0 = fresh_s(m.row0), last = fresh_s(m.nown - 1);
+#pragma unroll
+    for (int i = 0; i < RP; ++i)
+      if (res_on(left, i)) {
+        const int l = l0 + i * (kResNW * kWave);
+        f(i, l, l <= last, g0 + (l < last ? l : last));
+      }
+  };
+
+  // ---- reductions -------------------------------------------------------------
+  int nbar = 0, nred = 0;
+  int* cnt = V.ctl + 2 + m.team;
+  // Team barrier.  Exported stores are write-through: waiting for the store
+  // counter in every wavefront before the workgroup barrier makes them visible
+  // before thread 0 counts the arrival.  Bounded: a wait that gives up raises
+  // the abort flag, after which every wait of the launch ends.
+  auto barrier = [&]() -> bool {
+    ++nbar;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      const int target = nbar * T;
+      __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      int ok = 1;
+      long long t0 = 0;
+      for (int k = 0;; ++k) {
+        if (__hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= target) break;
+        if ((k & 15) == 15) {  // the clock and the abort flag every 16 polls
+          const long long now = (long long)wall_clock64();
+          if (t0 == 0) t0 = now;
+          if (__hip_atomic_load(V.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || k >= kResSpinMax ||
+              now - t0 > V.limit) {
+            __hip_atomic_store(V.ctl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(V.sticky, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ok = 0;
+            break;
+          }
+        }
+      }
+      *flag = ok;
+    }
+    __syncthreads();
+    return __builtin_amdgcn_readfirstlane(*flag) != 0;
+  };
+  // (Decisions taken from LDS values go through readfirstlane: the branches are
+  // uniform, and a divergent loop exit would copy every live register.)
+  // Sums two values over the system: wavefront butterfly, wavefronts in order,
+  // members by one butterfly over their ranks -- the same bits in every member.
+  auto sum = [&](double& s0, double& s1) -> bool {
+    s0 = wave_sum(s0);
+    s1 = wave_sum(s1);
+    if (lane == 0) {
+      red[2 * w] = s0;
+      red[2 * w + 1] = s1;
+    }
+    __syncthreads();
+    s0 = red[0];
+    s1 = red[1];
+#pragma unroll
+    for (int k = 1; k < kResNW; ++k) {
+      s0 += red[2 * k];
+      s1 += red[2 * k + 1];
+    }
+    if (T == 1) {
+      __syncthreads();
+      return true;
+    }
+    double* ps = V.part + (size_t)m.team * (4 * kResTeamMax) + (nred & 1) * (2 * kResTeamMax);
+    ++nred;
+    if (threadIdx.x == 0) {
+      st_agent(ps + 2 * m.rank, s0);
+      st_agent(ps + 2 * m.rank + 1, s1);
+    }
+    if (!barrier()) return false;
+    if (w == 0) {
+      double t0 = lane < T ? ld_agent(ps + 2 * lane) : 0.0, t1 = lane < T ? ld_agent(ps + 2 * lane + 1) : 0.0;
+      t0 = wave_sum(t0);
+      t1 = wave_sum(t1);
+      if (lane == 0) {
+        red[0] = t0;
+        red[1] = t1;
+      }
+    }
+    __syncthreads();
+    s0 = red[0];
+    s1 = red[1];
+    __syncthreads();
+    return true;
+  };
+
+  // ---- q = A v for v in LDS -----------------------------------------------------
+  auto unpack = [](const uint4& c, int u) {
+    const unsigned wd = u < 2 ? c.x : u < 4 ? c.y : u < 6 ? c.z : c.w;
+    return (u & 1) ? wd >> 16 : wd & 0xffffu;
+  };
+  // Slots past the slice's width re-read its last slot; their index is the zero
+  // entry.  Offsets are formed in scalar registers, the lane's part in one vector.
+  auto fetch = [&](int k0, int left, int g, int ln, uint4& c, double(&v)[8]) {
+    c = (V.lcol + (size_t)g * kWave)[ln];
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      v[u] = __builtin_nontemporal_load((V.val + (size_t)(k0 + (u < left ? u : left - 1)) * kWave) + ln);
+  };
+  auto accumulate = [&](const uint4& c, const double(&v)[8], double& acc) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) acc = fma(v[u], lds[unpack(c, u)], acc);
+  };
+  auto product = [&]() {
+    const int left = fresh_s(m.nsl - w), ln = fresh_v(lane);
+    const int kr = fresh_v(kreg), wr = fresh_v(wreg), gr = fresh_v(greg);
+    auto slot = [&](int i) { return __builtin_amdgcn_readlane(kr, i); };
+    auto width = [&](int i) { return __builtin_amdgcn_readlane(wr, i); };
+    auto group = [&](int i) { return __builtin_amdgcn_readlane(gr, i); };
+    if constexpr (W8) {
+      // the next slice's entries are in flight while this one's are used
+      uint4 c[2];
+      double v[2][8];
+      if (left > 0) fetch(slot(0), width(0), group(0), ln, c[0], v[0]);
+#pragma unroll
+      for (int i = 0; i < RP; ++i) {
+        if (res_on(left, i)) {
+          if (i + 1 < RP && res_on(left, i + 1))
+            fetch(slot(i + 1), width(i + 1), group(i + 1), ln, c[(i + 1) & 1], v[(i + 1) & 1]);
+          double acc = 0.0;
+          accumulate(c[i & 1], v[i & 1], acc);
+          q[i] = acc;
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < RP; ++i) {
+        if (res_on(left, i)) {
+          const int k0 = slot(i), g0 = group(i), wd = width(i);
+          double acc = 0.0;
+          for (int k = 0; k < wd; k += 8) {
+            uint4 c;
+            double v[8];
+            fetch(k0 + k, wd - k, g0 + k / 8, ln, c, v);
+            accumulate(c, v, acc);
+          }
+          q[i] = acc;
+        }
+      }
+    }
+  };
+  const int* halo = V.halo + m.halo_off;
+  // LDS <- the vector whose own rows are f(i, g) and whose halo rows are in `src`
+  auto load_vec = [&](auto&& f, const double* src) {
+    for_rows([&](int i, int l, bool, int g) { lds[l] = f(i, g); });
+    for (int h = threadIdx.x; h < m.nhalo; h += kResNT) lds[own + h] = src ? ld_agent(src + halo[h]) : 0.0;
+    __syncthreads();
+  };
+  auto fail = [&]() {
+    if (threadIdx.x == 0)
+      __hip_atomic_fetch_max(a.out.status + m.sys, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  };
+  auto store_x = [&](bool zero) {
+    for_rows([&](int i, int, bool real, int g) {
+      if (real) a.x[g] = zero ? 0.0 : x[i];
+    });
+  };
+  auto finish = [&](int iters, double resid, int st) {
+    if (threadIdx.x == 0) {
+      if (m.rank == 0) {
+        a.out.iters[m.sys] = iters;
+        a.out.resid[m.sys] = resid;
+      }
+      __hip_atomic_fetch_max(a.out.status + m.sys, st, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+  };
+  if (threadIdx.x == 0) lds[own + m.nhalo] = 0.0;
+  const bool init = a.init_x != 0;
+  for_rows([&](int i, int, bool, int g) { x[i] = init ? 0.0 : a.x[g]; });
+  load_vec([&](int i, int) { return x[i]; }, init ? nullptr : a.x);
+  // One loop body holds the only matrix product and the only preconditioner
+  // pass.  LDS holds x when `resid_step` (the initial residual and the
+  // replacement every 200 iterations), else p.
+  bool resid_step = true;
+  double B2 = 0.0, rho = 0.0, beta = 0.0, resid = 1.0;
+  int it = 0;
+  for (;;) {
+    product();
+    double rr = 0.0, rz = 0.0, none = 0.0;
+    double alpha = 0.0;
+    if (!resid_step) {
+      for_rows([&](int i, int l, bool, int) { rr = fma(lds[l], q[i], rr); });
+      if (!sum(rr, none)) return fail();
+      alpha = rho / rr;  // (p, q)
+      rr = 0.0;
+      for_rows([&](int i, int l, bool, int) { x[i] = fma(alpha, lds[l], x[i]); });
+      if (it % kResIterRR == 0) {
+        // the true residual: p is set aside while LDS holds x
+        for_rows([&](int i, int l, bool real, int g) {
+          if (real) {
+            st_agent(a.p + g, lds[l]);
+            st_agent(a.x + g, x[i]);
+          }
+        });
+        if (T > 1) {
+          if (!barrier()) return fail();
+        } else {
+          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __syncthreads();
+        }
+        load_vec([&](int i, int) { return x[i]; }, a.x);
+        resid_step = true;
+        continue;
+      }
+    }
+    // r, then z = M^-1 r (kept in q's registers), (r, r), (r, z); z of exported slices goes out
+    for_rows([&](int i, int, bool real, int g) {
+      const double d = a.precond ? V.dinv[g] : 1.0;
+      double rv = resid_step ? a.b[g] - q[i] : fma(-alpha, q[i], r[i]);
+      rv = real ? rv : 0.0;
+      const double zv = a.precond ? d * rv : rv;
+      r[i] = rv;
+      q[i] = zv;
+      rr = fma(rv, rv, rr);
+      rz = fma(rv, zv, rz);
+      if ((exports >> i) & 1)
+        if (real) st_agent(a.z + g, zv);
+    });
+    if (resid_step) {
+      __syncthreads();  // LDS reads of the product are done
+      load_vec([&](int, int g) { return it > 0 ? ld_agent(a.p + g) : 0.0; }, it > 0 ? a.p : nullptr);
+      resid_step = false;
+    }
+    if (!sum(rr, rz)) return fail();
+    if (it == 0) {
+      B2 = rr;
+      if (__builtin_amdgcn_readfirstlane(B2 == 0.0)) {  // mat_converge.f90:40-48
+        store_x(true);
+        return finish(0, 0.0, 2);
+      }
+    } else {
+      resid = sqrt(rr / B2);
+      if (a.hist && m.rank == 0 && threadIdx.x == 0) a.hist[it] = resid;
+      const bool conv = __builtin_amdgcn_readfirstlane(resid < a.tol);
+      if (conv || it >= a.max_iter) {
+        store_x(false);
+        return finish(it, resid, conv ? 0 : 1);
+      }
+      beta = rz / rho;
+    }
+    rho = rz;
+    ++it;
+    // p = z + beta p (CG.f90:80-84; p = 0 before the first iteration), own rows and halo copies
+    constexpr int HU = 4;
+    for (int h0 = threadIdx.x; h0 < m.nhalo; h0 += HU * kResNT) {
+      double zv[HU];
+#pragma unroll
+      for (int u = 0; u < HU; ++u) {
+        const int h = h0 + u * kResNT;
+        zv[u] = ld_agent(a.z + halo[h < m.nhalo ? h : h0]);
+      }
+#pragma unroll
+      for (int u = 0; u < HU; ++u) {
+        const int h = h0 + u * kResNT;
+        if (h < m.nhalo) lds[own + h] = fma(beta, lds[own + h], zv[u]);
+      }
+    }
+    for_rows([&](int i, int l, bool, int) { lds[l] = fma(beta, lds[l], q[i]); });
+    __syncthreads();
+  }
+}
+
+// Persistent: workgroups take members in order from one counter.  A team's
+// members are consecutive, so at most one team is incomplete at any time and a
+// member waiting for a teammate that has not started waits only for running
+// workgroups to finish their own complete teams.
+template <int RP>
+__global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP <= kResRowsSmall ? 4 : 2)))
+    k_res_cg(ResView V, ResArgs a) {
+  extern __shared__ double res_lds[];
+  __shared__ double red[2 * kResNW];
+  __shared__ int sh[2];
+  for (;;) {
+    if (threadIdx.x == 0) sh[0] = __hip_atomic_fetch_add(V.ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    const int k = __builtin_amdgcn_readfirstlane(sh[0]);
+    if (k >= V.nmem) break;
+    const ResMember m = V.mem[k];
+    if (m.w8) res_cg<RP, true>(V, m, a, res_lds, red, sh + 1);
+    else res_cg<RP, false>(V, m, a, res_lds, red, sh + 1);
+    __syncthreads();
+  }
+}
+
+// One system of a plan.
+struct ResSystem {
+  int slice0, nsl, row0, rows;
+  double work;  // estimated work of the system (any unit)
+};
+
+// Members, halo lists and LDS indices of a set of systems (per pattern).
+struct ResPlan {
+  bool fits = false;
+  int nmem = 0, nteam = 0, grid = 0, rp = 0;
+  size_t lds_bytes = 0;
+  double ticks_per_s = 0;
+  DevArray<unsigned char> mem, expf, lcol;
+  DevArray<int> halo, g_ptr, ctl, sticky;
+  DevArray<double> part;
+};
+
+// slice_ptr: host slot offsets of every slice; d_slice_ptr / d_col: the device
+// arrays (global 0-based columns); rowlen (per SELL row) or rowptr (per row)
+// gives the row lengths.  Plan.fits is false when a system needs more than
+// kResTeamMax members or a member's rows and halo exceed LDS.
+int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
+                   const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int team_limit,
+                   hipStream_t s);
+// Zeroes the counters and enqueues the solver (both capturable).
+int res_launch(const ResPlan& plan, const int* d_slice_ptr, const double* val, const double* dinv, const ResArgs& a,
+               int nsys, double wait_s, hipStream_t s);
+// 1 when a team wait gave up in any launch since the last call (synchronises).
+int res_aborted(ResPlan& plan, int* aborted, hipStream_t s);
+
+}  // namespace mh

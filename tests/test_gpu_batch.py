@@ -239,3 +239,119 @@ def test_batch_team_no_preconditioner_and_iteration_limit(cfg):
             assert status[k] == 1 and iters[k] == 12, (k, status[k], iters[k])
         assert np.linalg.norm(xk - xo) / np.linalg.norm(xo) <= 1e-6, k
     assert limited > 0
+
+
+# ---- the on-chip solver (configuration 15) -----------------------------------
+ON_CHIP = 15
+
+
+def _concat(mats):
+    n = nnz = 0
+    idx, item, A, rows = [np.zeros(1, np.int64)], [], [], [0]
+    for m in mats:
+        idx.append(np.asarray(m.index[1:], np.int64) + nnz)
+        item.append(np.asarray(m.item, np.int64) + n)
+        A.append(m.A)
+        nnz += len(m.item)
+        n += m.n
+        rows.append(n)
+    return (Matrix(n, n, 1, np.concatenate(idx).astype(np.int32), np.concatenate(item).astype(np.int32),
+                   np.concatenate(A)).ensure_dof_index(), np.array(rows, np.int64))
+
+
+def _irregular(n, far, seed):
+    """Symmetric diagonally dominant rows of 1 to about 20 entries, some `far` rows apart."""
+    rng = np.random.default_rng(seed)
+    i = rng.integers(0, n, 4 * n)
+    d = np.where(rng.uniform(size=4 * n) < 0.3, far, rng.integers(1, 40, 4 * n))
+    j = i + d
+    keep = (j < n) & (i % 5 != 0) & (j % 5 != 0)            # every fifth row holds its diagonal alone
+    key = np.unique(i[keep] * n + j[keep])
+    i, j = key // n, key % n
+    v = -rng.uniform(0.1, 1.0, len(i))
+    rows = np.concatenate([i, j, np.arange(n)])
+    cols = np.concatenate([j, i, np.arange(n)])
+    off = np.bincount(np.concatenate([i, j]), weights=np.abs(np.concatenate([v, v])), minlength=n)
+    vals = np.concatenate([v, v, off + 0.05])
+    order = np.lexsort((cols, rows))
+    index = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    return Matrix(n, n, 1, index, (cols[order] + 1).astype(np.int32), vals[order]).ensure_dof_index()
+
+
+# one row, whole and partial slices, the last size solved whole and the first split, rows of 1..20 entries
+# (more and less than eight slots), a halo reaching across the system
+@pytest.mark.parametrize("precond", [0, 1])
+@pytest.mark.parametrize("sizes", [(1, 63, 64, 65), (2048, 2049, 517), (9000,), (30000, 14000, 700)])
+def test_on_chip_irregular_systems(sizes, precond):
+    mat, sys_row = _concat([_irregular(n, max(1, n // 3), n) for n in sizes])
+    b = W.uniform_vector(mat.n, seed=4)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
+    B = api.DeviceBatch(mat, sys_row)
+    B.set_config(ON_CHIP)
+    sch = B.schedule(ON_CHIP)
+    assert sch["split"] == 1 and (sch["teams"] > 0) == (max(sizes) > 2048), sch
+    iters, resid, status = B.solve(db, dx, _prm(precond=precond))
+    x = dx.numpy()
+    _check_against_oracle(mat, sys_row, b, x, iters, resid, status, precond=precond)
+    for _ in range(3):                               # graph replays: same bits
+        it1, r1, s1 = B.solve(db, dx, _prm(precond=precond))
+        assert np.array_equal(x, dx.numpy()) and np.array_equal(iters, it1) and np.array_equal(status, s1)
+
+
+def test_on_chip_teams_residual_replacement_start_vector_and_limits():
+    # a team of the largest kind of member, past iteration 200; a zero right-hand side; a start vector;
+    # a limit of 12 iterations
+    edges = [56, 5, 30, 12, 20]
+    mat, sys_row = W.poisson_batch(edges=edges)
+    b = W.uniform_vector(mat.n, seed=21)
+    b[sys_row[1]:sys_row[2]] = 0.0
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
+    B = api.DeviceBatch(mat, sys_row)
+    assert B.schedule(ON_CHIP)["teams"] >= 2         # also the default of a batch that fits
+    iters, resid, status = B.solve(db, dx, _prm())
+    assert iters[0] > 200
+    x = dx.numpy()
+    _check_against_oracle(mat, sys_row, b, x, iters, resid, status, zero=(1,))
+    x0 = W.uniform_vector(mat.n, seed=9)
+    prm = _prm()
+    prm.Iarray[api.MONOLIS_PRM_I_IS_INIT_X] = 0
+    dx.upload(x0)
+    it2, r2, s2 = B.solve(db, dx, prm)
+    assert np.all(s2 == 0)
+    x2 = dx.numpy()
+    for k in range(B.nsys):
+        s = slice(sys_row[k], sys_row[k + 1])
+        if k != 1:
+            assert np.linalg.norm(x2[s] - x[s]) <= 1e-5 * np.linalg.norm(x[s])
+    it3, r3, s3 = B.solve(db, dx, _prm(max_iter=12))
+    x3 = dx.numpy()
+    for k in (0, 2, 3, 4):
+        s = slice(sys_row[k], sys_row[k + 1])
+        xo, st, I, R = oracle.solve(_system(mat, sys_row, k), b[s], precond=1, max_iter=12)
+        assert s3[k] == (1 if st else 0) and np.linalg.norm(x3[s] - xo) <= 1e-6 * np.linalg.norm(xo)
+
+
+def test_on_chip_batch_that_does_not_fit_runs_another_configuration():
+    mat, sys_row = _concat([_irregular(450000, 1000, 3), _irregular(300, 7, 4)])
+    b = W.uniform_vector(mat.n, seed=4)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
+    B = api.DeviceBatch(mat, sys_row)
+    assert B.schedule(ON_CHIP)["split"] != 1
+    B.set_config(ON_CHIP)
+    iters, resid, status = B.solve(db, dx, _prm())
+    _check_against_oracle(mat, sys_row, b, dx.numpy(), iters, resid, status)
+
+
+def test_on_chip_wait_limit_gives_up_cleanly():
+    mat, sys_row = W.poisson_batch(edges=[30, 24, 9])
+    b = W.uniform_vector(mat.n, seed=4)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
+    B = api.DeviceBatch(mat, sys_row)
+    B.set_wait_limit(0.0)
+    try:
+        B.solve(db, dx, _prm())
+    except RuntimeError as e:
+        assert "gave up" in str(e)
+    B.set_wait_limit(5.0)
+    iters, resid, status = B.solve(db, dx, _prm())
+    _check_against_oracle(mat, sys_row, b, dx.numpy(), iters, resid, status)
