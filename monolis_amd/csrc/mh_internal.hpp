@@ -126,6 +126,8 @@ struct VBlock {
 // Device matrix: SELL-64 pattern + FP64 (and optionally FP32) values, plus the
 // CSR arrays kept for the preconditioner setup, transposes and gradients.
 // ---------------------------------------------------------------------------
+struct ResPlan;  // on-chip solver's members (mh_resident.hpp)
+
 struct Matrix {
   int n = 0, np = 0, nz = 0, b = 0;
   int nslices = 0;
@@ -153,6 +155,7 @@ struct Matrix {
   DevArray<int> tperm, tiperm;
   bool transpose_stale = false;   // values of A changed since the transpose was filled
   VBlock* vb = nullptr;           // non-null for variable block sizes
+  ResPlan* res = nullptr;         // built by the first solve that may run on chip
   // complex matrices (monolis's *_C path): values in valz instead of val64,
   // complex block-Jacobi factors in Dz (same structure-of-arrays layout as D64)
   bool is_complex = false;

@@ -18,6 +18,7 @@
 
 #include "mh_internal.hpp"
 #include "mh_launch.hpp"
+#include "mh_resident.hpp"
 #include "mh_vblock.hpp"
 
 namespace mh {
@@ -1283,10 +1284,77 @@ size_t cg_bytes(const Matrix& M, int nvec, int max_iter) {
 }
 
 
+// The on-chip CG on a scalar system (mh_resident.hpp): one launch instead of
+// three per iteration.  *ran stays false when the system does not fit, or when
+// a team's wait gave up (x is then as it was); the launch-per-step solver
+// follows.  Solves with a time split take that one too: it times its steps.
+int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, double* x, Workspace& W,
+               SolveResult* out, bool* ran, hipStream_t s) {
+  *ran = false;
+  if (M.n < 1 || M.n != M.np || P.max_iter < 1 || active_ktimer()) return 0;
+  if ((long long)M.nslices > (long long)kResTeamMax * kResRowsLarge * kResNW) return 0;
+  if (!M.res) {
+    M.res = new ResPlan();
+    std::vector<int> sp((size_t)M.nslices + 1);
+    MH_HIP(hipMemcpyAsync(sp.data(), M.slice_ptr.p, sizeof(int) * sp.size(), hipMemcpyDeviceToHost, s));
+    MH_HIP(hipStreamSynchronize(s));
+    MH_TRY(res_plan_build(*M.res, {ResSystem{0, M.nslices, 0, M.n, 1.0}}, sp.data(), M.nslices, M.slice_ptr.p,
+                          M.col.p, nullptr, M.rowptr.p, cu_count(), s));
+  }
+  // With the matrix in registers always; otherwise while a member streams at
+  // most 300 KB per iteration (about 10 us from one CU).
+  if (!M.res->fits || (!M.res->mr && (double)M.nslots * kWave * 10.0 > 300e3 * M.res->nmem)) return 0;
+  struct Result {
+    int iter, status;
+    double resid;
+  } h{0, 3, 0.0};
+  const size_t m = (size_t)M.n;
+  MH_TRY(W.ensure(4 * (m * sizeof(double) + 256) + ((size_t)P.max_iter + 2) * sizeof(double) + 1024));
+  Carve cv{W.raw.p};
+  double* z = cv.take<double>(m);
+  double* p = cv.take<double>(m);
+  double* xe = cv.take<double>(m);
+  double* x0 = cv.take<double>(m);
+  double* hist = cv.take<double>((size_t)P.max_iter + 2);
+  Result* d = cv.take<Result>(1);
+  if (!P.init_x) MH_HIP(hipMemcpyAsync(x0, x, m * sizeof(double), hipMemcpyDeviceToDevice, s));
+  const ResArgs a{b, x, z, p, xe, {&d->iter, &d->resid, &d->status}, P.keep_hist ? hist : nullptr, P.max_iter, P.tol,
+                  P.init_x, prec ? 1 : 0};
+  MH_TRY(res_launch(*M.res, M.slice_ptr.p, M.val64.p, prec ? M.D64.p : nullptr, a, 1, 5.0, s));
+  MH_HIP(hipMemcpyAsync(&h, d, sizeof(Result), hipMemcpyDeviceToHost, s));
+  MH_HIP(hipStreamSynchronize(s));
+  if (h.status < 0 || h.status > 2) {
+    int gave_up = 0;
+    MH_TRY(res_aborted(*M.res, &gave_up, s));
+    if (!P.init_x) MH_HIP(hipMemcpyAsync(x, x0, m * sizeof(double), hipMemcpyDeviceToDevice, s));
+    return 0;
+  }
+  out->hist.clear();
+  out->zero_rhs = h.status == 2;
+  out->converged = h.status != 1;
+  out->iter = h.status == 2 ? -1 : h.iter;
+  out->resid = h.resid;
+  if (P.keep_hist && out->iter > 0) {
+    out->hist.resize((size_t)out->iter + 1);
+    out->hist[0] = 0.0;
+    MH_HIP(hipMemcpyAsync(out->hist.data() + 1, hist + 1, sizeof(double) * (size_t)out->iter, hipMemcpyDeviceToHost, s));
+    MH_HIP(hipStreamSynchronize(s));
+  }
+  *ran = true;
+  return 0;
+}
+
 template <typename T, int B, bool PREC>
 int cg_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& W, SolveResult* out, hipStream_t s) {
   Context* c = nullptr;
   MH_TRY(context(&c));
+  if constexpr (B == 1 && sizeof(T) == 8) {
+    if (!PREC || !M.vb) {
+      bool ran = false;
+      MH_TRY(cg_on_chip(M, P, PREC, b, x, W, out, &ran, s));
+      if (ran) return 0;
+    }
+  }
   const size_t vec = (size_t)M.np * B;
   MH_TRY(W.ensure(cg_bytes<T>(M, 5, P.max_iter)));
   Carve cv{W.raw.p};

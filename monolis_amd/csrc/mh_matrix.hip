@@ -10,6 +10,7 @@
 
 #include "mh_internal.hpp"
 #include "mh_launch.hpp"
+#include "mh_resident.hpp"
 
 namespace mh {
 
@@ -444,6 +445,7 @@ static int grid_1d(size_t m) {
 Matrix::~Matrix() {
   delete transpose;
   delete vb;
+  delete res;
 }
 
 template <typename TV>

@@ -102,22 +102,24 @@ __global__ void __launch_bounds__(kResNT) k_res_build(ResMember* mem, const int*
 }
 
 // Per-launch reset (a kernel, so that a captured graph holds no memset nodes).
-__global__ void k_res_reset(int nsys, int* iters, double* resid, int* status, int* ctl, int nctl) {
+__global__ void k_res_reset(int nsys, int* iters, double* resid, int* status, int* ctl, unsigned long long* part,
+                            int npart) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nsys) {
     iters[i] = -1;
     resid[i] = 0.0;
     status[i] = -1;
   }
-  if (i < nctl) ctl[i] = 0;
+  if (i < 2) ctl[i] = 0;
+  if (i < npart) part[i] = 0;  // no tag of an earlier launch
 }
 
-template <int RP>
+template <int RP, bool MR>
 int occupancy(size_t lds, int* per_cu) {
-  MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_res_cg<RP>), hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)lds));
+  auto* k = &k_res_cg<RP, MR>;
+  MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   *per_cu = 0;
-  MH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k_res_cg<RP>, kResNT, lds));
+  MH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k, kResNT, lds));
   return 0;
 }
 
@@ -145,12 +147,14 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
     if (q.rows == 0) return 0;
     const int need = (q.nsl + kResRowsLarge * kResNW - 1) / (kResRowsLarge * kResNW);
     // More members than capacity asks for, while the system's share of the
-    // workgroups allows: a barrier pair and the halo cost about 4 us per
-    // iteration, a 512-row step of a member about 0.5 us, so a member keeps at
-    // least two steps and systems of up to four stay whole.
+    // workgroups allows: down to one row per thread (7-point systems, us per
+    // iteration with 64 / 128 members: 48^3 10.3 / 8.1, 64^3 19.7 / 11.2, 78^3
+    // 34.8 / 19.8; 32^3 is flat from 32 to 128 at 7.0-7.3).  Up to four rows per
+    // thread one workgroup alone is faster (10^3: 4.0 against 5.7 with four
+    // members, 12^3: 4.5 against 6.0): a team's two exchanges cost about 1 us each.
     const int fair = (int)((double)team_limit * q.work / std::max(W, 1e-300));
-    int T = std::max(need, std::min(std::min(kResTeamMax, fair), q.nsl / (2 * kResNW)));
-    if (need == 1 && q.nsl <= 4 * kResNW) T = 1;
+    int T = std::max(need, std::min(std::min(kResTeamMax, fair), q.nsl / kResNW));
+    if (need == 1 && q.nsl <= kResRowsMini * kResNW) T = 1;
     T = std::max(T, 1);
     if (T > kResTeamMax) return 0;
     tasks.push_back(Task{(int)k, T, ((double)q.rows / T + 1500.0) * std::cbrt((double)q.rows)});
@@ -203,8 +207,8 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
   MH_TRY(plan.lcol.alloc((size_t)std::max(groups, 1LL) * kWave * sizeof(uint4)));
   MH_TRY(plan.halo.alloc((size_t)std::max(halo_total, 1LL)));
   MH_TRY(plan.g_ptr.alloc((size_t)nslices + 1));
-  MH_TRY(plan.ctl.alloc((size_t)2 + nteam));
-  MH_TRY(plan.part.alloc((size_t)std::max(nteam, 1) * 4 * kResTeamMax));
+  MH_TRY(plan.ctl.alloc(2));
+  MH_TRY(plan.part.alloc((size_t)std::max(nteam, 1) * 8 * kResTeamMax));
   MH_TRY(plan.sticky.alloc(2));  // [1]: a halo that does not fit (build only)
   MH_TRY(upload(plan.mem.p, mem.data(), mem.size() * sizeof(ResMember), s));
   MH_TRY(upload(plan.g_ptr.p, g_ptr.data(), sizeof(int) * ((size_t)nslices + 1), s));
@@ -221,14 +225,26 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
   MH_HIP(hipMemcpyAsync(bad, plan.sticky.p, 2 * sizeof(int), hipMemcpyDeviceToHost, s));
   MH_HIP(hipStreamSynchronize(s));
   if (bad[1]) return 0;
-  int lds = 0;
-  for (const ResMember& m : mem) lds = std::max(lds, m.nsl * kWave + m.nhalo + 1);
-  plan.lds_bytes = (size_t)lds * sizeof(double);
+  // Members of at most kResRowsSmall rows per thread: the matrix in registers
+  // too (and x in LDS) if every row has at most 8 entries, else two workgroups
+  // per CU.
+  const bool small = max_nsl <= kResRowsSmall * kResNW;
+  int lds = 0, lds_mr = 0;
+  bool w8 = true;
+  for (const ResMember& m : mem) {
+    lds = std::max(lds, m.nsl * kWave + m.nhalo + 1);
+    lds_mr = std::max(lds_mr, 2 * m.nsl * kWave + m.nhalo + 1);
+    w8 = w8 && m.w8;
+  }
+  const bool mini = max_nsl <= kResRowsMini * kResNW && w8;
+  plan.mr = mini || (small && w8 && lds_mr <= kResLds);
+  plan.lds_bytes = (size_t)(plan.mr && !mini ? lds_mr : lds) * sizeof(double);
   int per_cu = 0;
-  // two workgroups per CU where every member fits half of one
-  plan.rp = max_nsl <= kResRowsSmall * kResNW && plan.lds_bytes <= ((size_t)79 << 10) ? kResRowsSmall : kResRowsLarge;
-  if (plan.rp == kResRowsSmall) MH_TRY(occupancy<kResRowsSmall>(plan.lds_bytes, &per_cu));
-  else MH_TRY(occupancy<kResRowsLarge>(plan.lds_bytes, &per_cu));
+  plan.rp = mini ? kResRowsMini : plan.mr || (small && plan.lds_bytes <= ((size_t)79 << 10)) ? kResRowsSmall : kResRowsLarge;
+  if (mini) MH_TRY((occupancy<kResRowsMini, true>(plan.lds_bytes, &per_cu)));
+  else if (plan.mr) MH_TRY((occupancy<kResRowsSmall, true>(plan.lds_bytes, &per_cu)));
+  else if (plan.rp == kResRowsSmall) MH_TRY((occupancy<kResRowsSmall, false>(plan.lds_bytes, &per_cu)));
+  else MH_TRY((occupancy<kResRowsLarge, false>(plan.lds_bytes, &per_cu)));
   if (per_cu < 1) return 0;
   plan.grid = std::min(plan.nmem, per_cu * cu_count());
   int dev = 0, khz = 0;
@@ -241,15 +257,17 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
 
 int res_launch(const ResPlan& plan, const int* d_slice_ptr, const double* val, const double* dinv, const ResArgs& a,
                int nsys, double wait_s, hipStream_t s) {
-  const int nctl = 2 + plan.nteam;
-  k_res_reset<<<(std::max(nsys, nctl) + kBlock - 1) / kBlock, kBlock, 0, s>>>(nsys, a.out.iters, a.out.resid,
-                                                                             a.out.status, plan.ctl.p, nctl);
+  const int npart = plan.nteam * 8 * kResTeamMax;
+  k_res_reset<<<(std::max(nsys, npart + 2) + kBlock - 1) / kBlock, kBlock, 0, s>>>(
+      nsys, a.out.iters, a.out.resid, a.out.status, plan.ctl.p, plan.part.p, npart);
   MH_HIP(hipGetLastError());
   const ResView V{plan.nmem, (const ResMember*)plan.mem.p, d_slice_ptr, plan.g_ptr.p, val, (const uint4*)plan.lcol.p,
                   plan.expf.p, dinv, plan.halo.p, plan.ctl.p, plan.part.p, (long long)(plan.ticks_per_s * wait_s),
                   plan.sticky.p};
-  if (plan.rp == kResRowsSmall) k_res_cg<kResRowsSmall><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
-  else k_res_cg<kResRowsLarge><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  if (plan.rp == kResRowsMini) k_res_cg<kResRowsMini, true><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  else if (plan.mr) k_res_cg<kResRowsSmall, true><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  else if (plan.rp == kResRowsSmall) k_res_cg<kResRowsSmall, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  else k_res_cg<kResRowsLarge, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
   MH_HIP(hipGetLastError());
   return 0;
 }

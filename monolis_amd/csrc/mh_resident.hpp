@@ -8,13 +8,19 @@
 // entry -- and the preconditioner's 8 bytes per row: about 80 bytes per row of a
 // 7-point system against 190 with the vectors in memory.  512 Poisson systems of
 // 10^3..40^3 rows: 51.1 -> 19.0 ms, 1.377e9 row-iterations at 72 G/s (5.8 TB/s of
-// those bytes): bound by the matrix stream.
+// those bytes): bound by the matrix stream.  A single 32^3 system: 1.93 -> 0.77
+// ms (17.7 -> 7.0 us per iteration, three launches before): bound by the two
+// exchanges and the halo loads, about 1 us each, and the sums' serial chains.
 //
 // Team members exchange two things, through agent-scope stores and loads that
 // bypass the XCD's L2 (no cache write-back or invalidation): the partial sums of
 // the two reductions of an iteration, and z of the rows some other member
 // reads.  Every member updates its copy of a halo row's p as its owner does,
 // p = z + beta p, so p itself is never exchanged.
+//
+// Members of at most kResRowsSmall * 512 rows of up to 8 entries also keep their
+// part of the matrix in registers (MR): an iteration then touches no memory but
+// the exchange.
 #pragma once
 
 #include <memory>
@@ -27,12 +33,13 @@ namespace mh {
 
 constexpr int kResNT = 512;                 // threads per member: two wavefronts per SIMD, 256 VGPRs each
 constexpr int kResNW = kResNT / kWave;
-constexpr int kResTeamMax = 32;             // workgroups per team at most
-constexpr int kResLds = 20352;              // doubles of LDS for p (159 KB of the CU's 160)
+constexpr int kResTeamMax = 128;            // workgroups per team at most (one wavefront polls 4 words of each)
+constexpr int kResLds = 20320;              // doubles of LDS for p (158.75 KB of the CU's 160)
 constexpr int kResSpinMax = 1 << 24;        // polls of one team wait at most (a bound that needs no clock)
 constexpr int kResIterRR = 200;             // residual replacement (CG.f90:91-95)
 constexpr int kResRowsLarge = 26;           // RP: 13,312 rows per member (150 VGPRs of vectors)
-constexpr int kResRowsSmall = 8;            // RP: 4,096 rows, two workgroups per CU
+constexpr int kResRowsMini = 4;             // RP: 2,048 rows
+constexpr int kResRowsSmall = 8;            // RP: 4,096 rows (with the matrix in registers: 208 VGPRs of data)
 
 struct ResMember {
   int sys, rank, T, team;
@@ -54,8 +61,8 @@ struct ResView {
   const unsigned char* expf;  // per slice: some other member reads a row of it
   const double* dinv;     // diagonal preconditioner per row
   const int* halo;        // global rows, per member
-  int* ctl;               // [0] next member, [1] abort flag, [2 + t] arrivals of team t
-  double* part;           // per team: 2 alternating sets x kResTeamMax x 2 partial sums
+  int* ctl;               // [0] next member, [1] abort flag
+  unsigned long long* part;  // per team: 2 alternating sets x kResTeamMax x 4 tagged halves of two sums
   long long limit;        // wall-clock ticks one wait may last
   int* sticky;            // set with the abort flag, cleared only by the host
 };
@@ -71,12 +78,20 @@ struct ResArgs {
   const double* b;
   double* x;
   double* z;       // exported z (written for exported slices only)
-  double* p;       // exported p (residual replacement only)
+  double* p;       // p and x during a residual replacement
+  double* xe;
   BatchOut out;
   double* hist;    // residual history of the only system, or null
   int max_iter;
   double tol;
   int init_x, precond;
+};
+
+// Workgroup state beside the LDS vector.
+struct ResShared {
+  double red[2][2 * kResNW];
+  double tot[2];
+  int ok, next;
 };
 
 __device__ __forceinline__ void st_agent(double* p, double v) {
@@ -109,16 +124,30 @@ __device__ __forceinline__ bool res_on(int left, int i) {
 }
 
 // One member's part of one system.
-template <int RP, bool W8>
-__device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, const ResArgs& a, double* lds, double* red,
-                                       int* flag) {
+template <int RP, bool W8, bool MR>
+__device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, const ResArgs& a, double* lds,
+                                       ResShared& sh) {
   const int lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
   const int own = m.nsl * kWave;  // LDS: own rows (whole slices), halo rows, one zero
   const int T = m.T;
-  double x[RP], r[RP], q[RP];     // row i of a thread: slice w + i*8 of the member, its lane
+  // Row i of a thread: slice w + i*8 of the member, its lane.  With eight rows of
+  // the matrix in registers x lies in LDS, behind p; with four the preconditioner
+  // and the first halo rows' numbers are held in registers too.
+  constexpr bool XL = MR && RP > kResRowsMini, KEEP = MR && RP <= kResRowsMini;
+  constexpr int HU = 4;  // halo rows per thread and step
+  double x[XL ? 1 : RP], r[RP], q[RP], dreg[KEEP ? RP : 1];
+  int hreg[KEEP ? HU : 1];
 #pragma unroll
-  for (int i = 0; i < RP; ++i) x[i] = r[i] = q[i] = 0.0;
+  for (int i = 0; i < RP; ++i) {
+    if constexpr (!XL) x[i] = 0.0;
+    r[i] = q[i] = 0.0;
+  }
+  double* xl = lds + own + m.nhalo + 1;
+  auto xv = [&](int i, int l) -> double& {
+    if constexpr (XL) return xl[l];
+    else return x[i];
+  };
   // lane i holds the slot and group offsets and the export bit of slice w + i*8
   int kreg = 0, wreg = 1, greg = 0;
   bool ereg = false;
@@ -146,51 +175,30 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
   };
 
   // ---- reductions -------------------------------------------------------------
-  int nbar = 0, nred = 0;
-  int* cnt = V.ctl + 2 + m.team;
-  // Team barrier.  Exported stores are write-through: waiting for the store
-  // counter in every wavefront before the workgroup barrier makes them visible
-  // before thread 0 counts the arrival.  Bounded: a wait that gives up raises
-  // the abort flag, after which every wait of the launch ends.
-  auto barrier = [&]() -> bool {
-    ++nbar;
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (threadIdx.x == 0) {
-      const int target = nbar * T;
-      __hip_atomic_fetch_add(cnt, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      int ok = 1;
-      long long t0 = 0;
-      for (int k = 0;; ++k) {
-        if (__hip_atomic_load(cnt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= target) break;
-        if ((k & 15) == 15) {  // the clock and the abort flag every 16 polls
-          const long long now = (long long)wall_clock64();
-          if (t0 == 0) t0 = now;
-          if (__hip_atomic_load(V.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || k >= kResSpinMax ||
-              now - t0 > V.limit) {
-            __hip_atomic_store(V.ctl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(V.sticky, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            ok = 0;
-            break;
-          }
-        }
-      }
-      *flag = ok;
-    }
-    __syncthreads();
-    return __builtin_amdgcn_readfirstlane(*flag) != 0;
-  };
-  // (Decisions taken from LDS values go through readfirstlane: the branches are
-  // uniform, and a divergent loop exit would copy every live register.)
   // Sums two values over the system: wavefront butterfly, wavefronts in order,
   // members by one butterfly over their ranks -- the same bits in every member.
+  // A member posts its sums as four 64-bit words, each half of a value with the
+  // number of the reduction as a tag; one wavefront of every member polls the
+  // words of all members and has the values as soon as the tags agree, without
+  // a counter or a second round trip.  Two alternating sets: a set is rewritten
+  // after a reduction that every member joined having read it.  The exported
+  // rows' write-through stores are waited for before the sums are posted, so a
+  // member that has read them may load those rows.
+  // Bounded: a wait that gives up raises the abort flag, after which every wait
+  // of the launch ends.  (Decisions taken from LDS values go through
+  // readfirstlane: the branches are uniform; a divergent loop exit would copy
+  // every live register.)
+  unsigned epoch = 0;
   auto sum = [&](double& s0, double& s1) -> bool {
+    ++epoch;
+    double* red = sh.red[epoch & 1];
     s0 = wave_sum(s0);
     s1 = wave_sum(s1);
     if (lane == 0) {
       red[2 * w] = s0;
       red[2 * w + 1] = s1;
     }
+    if (T > 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     s0 = red[0];
     s1 = red[1];
@@ -199,31 +207,67 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
       s0 += red[2 * k];
       s1 += red[2 * k + 1];
     }
-    if (T == 1) {
-      __syncthreads();
-      return true;
-    }
-    double* ps = V.part + (size_t)m.team * (4 * kResTeamMax) + (nred & 1) * (2 * kResTeamMax);
-    ++nred;
-    if (threadIdx.x == 0) {
-      st_agent(ps + 2 * m.rank, s0);
-      st_agent(ps + 2 * m.rank + 1, s1);
-    }
-    if (!barrier()) return false;
+    if (T == 1) return true;
     if (w == 0) {
-      double t0 = lane < T ? ld_agent(ps + 2 * lane) : 0.0, t1 = lane < T ? ld_agent(ps + 2 * lane + 1) : 0.0;
-      t0 = wave_sum(t0);
-      t1 = wave_sum(t1);
-      if (lane == 0) {
-        red[0] = t0;
-        red[1] = t1;
+      unsigned long long* ps = V.part + ((size_t)m.team * 2 + (epoch & 1)) * (4 * kResTeamMax);
+      if (lane < 4) {
+        const unsigned long long v = __double_as_longlong(lane < 2 ? s0 : s1);
+        const unsigned half = (lane & 1) ? (unsigned)(v >> 32) : (unsigned)v;
+        __hip_atomic_store(ps + 4 * m.rank + lane, (unsigned long long)epoch << 32 | half, __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
       }
+      constexpr int NL = 4 * kResTeamMax / kWave;  // words per lane
+      unsigned long long word[NL];
+      bool ok = true;
+      long long t0 = 0;
+      for (int k = 0;; ++k) {
+        bool all = true;
+#pragma unroll
+        for (int u = 0; u < NL; ++u) {
+          const int i = u * kWave + lane;
+          word[u] = (unsigned long long)epoch << 32;
+          if (u * kWave < 4 * T)
+            word[u] = __hip_atomic_load(ps + (i < 4 * T ? i : 0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+#pragma unroll
+        for (int u = 0; u < NL; ++u) all &= (unsigned)(word[u] >> 32) == epoch;
+        if (__all(all)) break;
+        if ((k & 15) == 15) {  // the clock and the abort flag every 16 polls
+          const long long now = (long long)wall_clock64();
+          if (t0 == 0) t0 = now;
+          if (__hip_atomic_load(V.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0 || k >= kResSpinMax ||
+              now - t0 > V.limit) {
+            __hip_atomic_store(V.ctl + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(V.sticky, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            ok = false;
+            break;
+          }
+        }
+      }
+      // lanes 4k, 4k+1 hold the halves of a member's first sum, 4k+2, 4k+3 of its second
+      double tot = 0.0;
+#pragma unroll
+      for (int u = 0; u < NL; ++u) {
+        const unsigned mine = (unsigned)word[u];
+        const unsigned other = (unsigned)__builtin_amdgcn_update_dpp(0, (int)mine, 0xB1, 0xf, 0xf, true);  // lane ^ 1
+        const unsigned long long v = (lane & 1) ? (unsigned long long)mine << 32 | other
+                                                : (unsigned long long)other << 32 | mine;
+        tot += u * kWave + lane < 4 * T ? __longlong_as_double(v) : 0.0;
+      }
+      tot += dpp_move<0x114>(tot);  // row_shr 4 and 8: lanes 12..15 of a row sum its four members
+      tot += dpp_move<0x118>(tot);
+      const double tot0 = (read_lane(tot, 12) + read_lane(tot, 28)) + (read_lane(tot, 44) + read_lane(tot, 60));
+      const double tot1 = (read_lane(tot, 14) + read_lane(tot, 30)) + (read_lane(tot, 46) + read_lane(tot, 62));
+      if (lane == 0) {
+        sh.tot[0] = tot0;
+        sh.tot[1] = tot1;
+      }
+      if (lane == 0) sh.ok = ok;
     }
     __syncthreads();
-    s0 = red[0];
-    s1 = red[1];
-    __syncthreads();
-    return true;
+    s0 = sh.tot[0];
+    s1 = sh.tot[1];
+    return __builtin_amdgcn_readfirstlane(sh.ok) != 0;
   };
 
   // ---- q = A v for v in LDS -----------------------------------------------------
@@ -243,8 +287,34 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
 #pragma unroll
     for (int u = 0; u < 8; ++u) acc = fma(v[u], lds[unpack(c, u)], acc);
   };
+  uint4 mc[MR ? RP : 1];
+  double mv[MR ? RP : 1][8];
+  if constexpr (MR) {
+    const int left = fresh_s(m.nsl - w);
+#pragma unroll
+    for (int i = 0; i < RP; ++i) {
+      mc[i] = make_uint4(0, 0, 0, 0);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) mv[i][u] = 0.0;
+      if (res_on(left, i))
+        fetch(__builtin_amdgcn_readlane(kreg, i), __builtin_amdgcn_readlane(wreg, i),
+              __builtin_amdgcn_readlane(greg, i), lane, mc[i], mv[i]);
+    }
+  }
   auto product = [&]() {
     const int left = fresh_s(m.nsl - w), ln = fresh_v(lane);
+    if constexpr (MR) {
+#pragma unroll
+      for (int i = 0; i < RP; ++i)
+        if (res_on(left, i)) {
+          uint4 c = mc[i];  // unpacked here, not once for the solve
+          asm volatile("" : "+v"(c.x), "+v"(c.y), "+v"(c.z), "+v"(c.w));
+          double acc = 0.0;
+          accumulate(c, mv[i], acc);
+          q[i] = acc;
+        }
+      return;
+    }
     const int kr = fresh_v(kreg), wr = fresh_v(wreg), gr = fresh_v(greg);
     auto slot = [&](int i) { return __builtin_amdgcn_readlane(kr, i); };
     auto width = [&](int i) { return __builtin_amdgcn_readlane(wr, i); };
@@ -282,19 +352,27 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
     }
   };
   const int* halo = V.halo + m.halo_off;
-  // LDS <- the vector whose own rows are f(i, g) and whose halo rows are in `src`
+  // LDS <- the vector whose own rows are f(i, l, g) and whose halo rows are in `src`
   auto load_vec = [&](auto&& f, const double* src) {
-    for_rows([&](int i, int l, bool, int g) { lds[l] = f(i, g); });
+    for_rows([&](int i, int l, bool, int g) { lds[l] = f(i, l, g); });
     for (int h = threadIdx.x; h < m.nhalo; h += kResNT) lds[own + h] = src ? ld_agent(src + halo[h]) : 0.0;
     __syncthreads();
   };
+  if constexpr (KEEP) {
+    for_rows([&](int i, int, bool, int g) { dreg[i] = a.precond ? V.dinv[g] : 1.0; });
+#pragma unroll
+    for (int u = 0; u < HU; ++u) {
+      const int h = threadIdx.x + u * kResNT;
+      hreg[u] = m.nhalo > 0 ? halo[h < m.nhalo ? h : 0] : 0;
+    }
+  }
   auto fail = [&]() {
     if (threadIdx.x == 0)
       __hip_atomic_fetch_max(a.out.status + m.sys, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   };
   auto store_x = [&](bool zero) {
-    for_rows([&](int i, int, bool real, int g) {
-      if (real) a.x[g] = zero ? 0.0 : x[i];
+    for_rows([&](int i, int l, bool real, int g) {
+      if (real) a.x[g] = zero ? 0.0 : xv(i, l);
     });
   };
   auto finish = [&](int iters, double resid, int st) {
@@ -308,8 +386,8 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
   };
   if (threadIdx.x == 0) lds[own + m.nhalo] = 0.0;
   const bool init = a.init_x != 0;
-  for_rows([&](int i, int, bool, int g) { x[i] = init ? 0.0 : a.x[g]; });
-  load_vec([&](int i, int) { return x[i]; }, init ? nullptr : a.x);
+  for_rows([&](int i, int l, bool, int g) { xv(i, l) = init ? 0.0 : a.x[g]; });
+  load_vec([&](int i, int l, int) { return xv(i, l); }, init ? nullptr : a.x);
   // One loop body holds the only matrix product and the only preconditioner
   // pass.  LDS holds x when `resid_step` (the initial residual and the
   // replacement every 200 iterations), else p.
@@ -325,29 +403,28 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
       if (!sum(rr, none)) return fail();
       alpha = rho / rr;  // (p, q)
       rr = 0.0;
-      for_rows([&](int i, int l, bool, int) { x[i] = fma(alpha, lds[l], x[i]); });
+      for_rows([&](int i, int l, bool, int) { xv(i, l) = fma(alpha, lds[l], xv(i, l)); });
       if (it % kResIterRR == 0) {
         // the true residual: p is set aside while LDS holds x
         for_rows([&](int i, int l, bool real, int g) {
           if (real) {
             st_agent(a.p + g, lds[l]);
-            st_agent(a.x + g, x[i]);
+            st_agent(a.xe + g, xv(i, l));
           }
         });
-        if (T > 1) {
-          if (!barrier()) return fail();
-        } else {
-          asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-          __syncthreads();
-        }
-        load_vec([&](int i, int) { return x[i]; }, a.x);
+        if (T == 1) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        double none2 = 0.0;
+        if (!sum(none, none2)) return fail();
+        load_vec([&](int i, int l, int) { return xv(i, l); }, a.xe);
         resid_step = true;
         continue;
       }
     }
     // r, then z = M^-1 r (kept in q's registers), (r, r), (r, z); z of exported slices goes out
     for_rows([&](int i, int, bool real, int g) {
-      const double d = a.precond ? V.dinv[g] : 1.0;
+      double d;
+      if constexpr (KEEP) d = dreg[i];
+      else d = a.precond ? V.dinv[g] : 1.0;
       double rv = resid_step ? a.b[g] - q[i] : fma(-alpha, q[i], r[i]);
       rv = real ? rv : 0.0;
       const double zv = a.precond ? d * rv : rv;
@@ -360,7 +437,7 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
     });
     if (resid_step) {
       __syncthreads();  // LDS reads of the product are done
-      load_vec([&](int, int g) { return it > 0 ? ld_agent(a.p + g) : 0.0; }, it > 0 ? a.p : nullptr);
+      load_vec([&](int, int, int g) { return it > 0 ? ld_agent(a.p + g) : 0.0; }, it > 0 ? a.p : nullptr);
       resid_step = false;
     }
     if (!sum(rr, rz)) return fail();
@@ -383,20 +460,23 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
     rho = rz;
     ++it;
     // p = z + beta p (CG.f90:80-84; p = 0 before the first iteration), own rows and halo copies
-    constexpr int HU = 4;
-    for (int h0 = threadIdx.x; h0 < m.nhalo; h0 += HU * kResNT) {
+    auto halo_step = [&](int h0, auto&& row) {
       double zv[HU];
 #pragma unroll
-      for (int u = 0; u < HU; ++u) {
-        const int h = h0 + u * kResNT;
-        zv[u] = ld_agent(a.z + halo[h < m.nhalo ? h : h0]);
-      }
+      for (int u = 0; u < HU; ++u) zv[u] = ld_agent(a.z + row(u, h0 + u * kResNT));
 #pragma unroll
       for (int u = 0; u < HU; ++u) {
         const int h = h0 + u * kResNT;
         if (h < m.nhalo) lds[own + h] = fma(beta, lds[own + h], zv[u]);
       }
+    };
+    auto listed = [&](int, int h) { return halo[h < m.nhalo ? h : 0]; };
+    int h0 = threadIdx.x;
+    if constexpr (KEEP) {
+      if (h0 < m.nhalo) halo_step(h0, [&](int u, int) { return hreg[u]; });
+      h0 += HU * kResNT;
     }
+    for (; h0 < m.nhalo; h0 += HU * kResNT) halo_step(h0, listed);
     for_rows([&](int i, int l, bool, int) { lds[l] = fma(beta, lds[l], q[i]); });
     __syncthreads();
   }
@@ -406,20 +486,23 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
 // members are consecutive, so at most one team is incomplete at any time and a
 // member waiting for a teammate that has not started waits only for running
 // workgroups to finish their own complete teams.
-template <int RP>
-__global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP <= kResRowsSmall ? 4 : 2)))
+template <int RP, bool MR>
+__global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP <= kResRowsSmall && !MR ? 4 : 2)))
     k_res_cg(ResView V, ResArgs a) {
   extern __shared__ double res_lds[];
-  __shared__ double red[2 * kResNW];
-  __shared__ int sh[2];
+  __shared__ ResShared sh;
   for (;;) {
-    if (threadIdx.x == 0) sh[0] = __hip_atomic_fetch_add(V.ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) sh.next = __hip_atomic_fetch_add(V.ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __syncthreads();
-    const int k = __builtin_amdgcn_readfirstlane(sh[0]);
+    const int k = __builtin_amdgcn_readfirstlane(sh.next);
     if (k >= V.nmem) break;
     const ResMember m = V.mem[k];
-    if (m.w8) res_cg<RP, true>(V, m, a, res_lds, red, sh + 1);
-    else res_cg<RP, false>(V, m, a, res_lds, red, sh + 1);
+    if constexpr (MR) {
+      res_cg<RP, true, true>(V, m, a, res_lds, sh);
+    } else {
+      if (m.w8) res_cg<RP, true, false>(V, m, a, res_lds, sh);
+      else res_cg<RP, false, false>(V, m, a, res_lds, sh);
+    }
     __syncthreads();
   }
 }
@@ -434,11 +517,12 @@ struct ResSystem {
 struct ResPlan {
   bool fits = false;
   int nmem = 0, nteam = 0, grid = 0, rp = 0;
+  bool mr = false;  // the members' matrix stays in registers
   size_t lds_bytes = 0;
   double ticks_per_s = 0;
   DevArray<unsigned char> mem, expf, lcol;
   DevArray<int> halo, g_ptr, ctl, sticky;
-  DevArray<double> part;
+  DevArray<unsigned long long> part;
 };
 
 // slice_ptr: host slot offsets of every slice; d_slice_ptr / d_col: the device

@@ -260,10 +260,11 @@ def _concat(mats):
 
 
 def _irregular(n, far, seed):
-    """Symmetric diagonally dominant rows of 1 to about 20 entries, some `far` rows apart."""
+    """Symmetric diagonally dominant rows of 1 to about 20 entries, some `far` rows apart (None: all at any distance)."""
     rng = np.random.default_rng(seed)
     i = rng.integers(0, n, 4 * n)
-    d = np.where(rng.uniform(size=4 * n) < 0.3, far, rng.integers(1, 40, 4 * n))
+    away = rng.integers(1, n, 4 * n) if far is None else far
+    d = np.where(rng.uniform(size=4 * n) < (1.0 if far is None else 0.3), away, rng.integers(1, 40, 4 * n))
     j = i + d
     keep = (j < n) & (i % 5 != 0) & (j % 5 != 0)            # every fifth row holds its diagonal alone
     key = np.unique(i[keep] * n + j[keep])
@@ -332,7 +333,7 @@ def test_on_chip_teams_residual_replacement_start_vector_and_limits():
 
 
 def test_on_chip_batch_that_does_not_fit_runs_another_configuration():
-    mat, sys_row = _concat([_irregular(450000, 1000, 3), _irregular(300, 7, 4)])
+    mat, sys_row = _concat([_irregular(600000, None, 3), _irregular(300, 7, 4)])
     b = W.uniform_vector(mat.n, seed=4)
     db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
     B = api.DeviceBatch(mat, sys_row)
