@@ -1414,7 +1414,7 @@ int cg_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& W, Sol
   // SpMV's partials.  Variable block sizes: diag_V runs after the update as
   // its own kernel and leaves (r, z) in parts_v.
   const bool vprec = PREC && B == 1 && M.vb != nullptr;
-  const int ntile_v = vprec ? rows_grid<T, 1>(M.vb->nb) : 0;
+  const int ntile_v = vprec ? rows_grid<T, kVPrecBS>(M.vb->nb) : 0;
   auto upd = [&](int it, int flags) -> int {
     const double* pre = (flags & (F_UPD | F_XONLY)) ? parts_s : nullptr;
     if constexpr (PREC && B == 1) {
@@ -1424,7 +1424,7 @@ int cg_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& W, Sol
         if (flags & F_XONLY) return 0;
         const VBlock& V = *M.vb;
         const T* DV = sizeof(T) == 8 ? (const T*)V.D64.p : (const T*)V.D32.p;
-        OpVPrec<T, true> vp{r, z, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0};
+        OpVPrec<T, true> vp{r, z, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0, V.maxb};
         return launch_rows<decltype(vp), false>(V.nb, vp, parts_v, s);
       }
     }
@@ -1507,10 +1507,10 @@ int gropcg_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& W,
       const VBlock& V = *M.vb;
       const T* DV = sizeof(T) == 8 ? (const T*)V.D64.p : (const T*)V.D32.p;
       if (dot) {
-        OpVPrec<T, true> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 2};
+        OpVPrec<T, true> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 2, V.maxb};
         return launch_rows(V.nb, vp, parts, s);
       }
-      OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0};
+      OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0, V.maxb};
       return launch_rows(V.nb, vp, nullptr, s);
     }
     (void)src;
@@ -1618,7 +1618,7 @@ int pipecg_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& W,
     if constexpr (PREC && B == 1) {
       const VBlock& V = *M.vb;
       const T* DV = sizeof(T) == 8 ? (const T*)V.D64.p : (const T*)V.D32.p;
-      OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0};
+      OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0, V.maxb};
       return launch_rows(V.nb, vp, nullptr, s);
     }
     (void)src;
@@ -1740,7 +1740,7 @@ int pipecr_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& W,
     if constexpr (PREC && B == 1) {
       const VBlock& V = *M.vb;
       const T* DV = sizeof(T) == 8 ? (const T*)V.D64.p : (const T*)V.D32.p;
-      OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0};
+      OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0, V.maxb};
       return launch_rows(V.nb, vp, nullptr, s);
     }
     (void)src;
@@ -1861,7 +1861,7 @@ int pipebicgstab_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspa
       if (vprec) {
         const VBlock& V = *M.vb;
         const T* DV = sizeof(T) == 8 ? (const T*)V.D64.p : (const T*)V.D32.p;
-        OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0};
+        OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0, V.maxb};
         return launch_rows(V.nb, vp, nullptr, s);
       }
     }
@@ -2038,7 +2038,7 @@ int bicgstab_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& 
     if constexpr (PREC && B == 1) {
       const VBlock& V = *M.vb;
       const T* DV = sizeof(T) == 8 ? (const T*)V.D64.p : (const T*)V.D32.p;
-      OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0};
+      OpVPrec<T, false> vp{src, dst, V.list.p, V.dof_index.p, V.doff.p, DV, st, 0, V.maxb};
       return launch_rows(V.nb, vp, nullptr, s);
     }
     (void)src;

@@ -379,7 +379,7 @@ int vdiag_apply(const Matrix& M, const T* x, T* y, hipStream_t s) {
   const VBlock& V = *M.vb;
   if (V.nb == 0) return 0;
   const T* D = sizeof(T) == 8 ? (const T*)V.D64.p : (const T*)V.D32.p;
-  OpVPrec<T, false> op{x, y, V.list.p, V.dof_index.p, V.doff.p, D, nullptr, 0};
+  OpVPrec<T, false> op{x, y, V.list.p, V.dof_index.p, V.doff.p, D, nullptr, 0, V.maxb};
   return launch_rows(V.nb, op, nullptr, s);
 }
 template int vdiag_apply<double>(const Matrix&, const double*, double*, hipStream_t);
