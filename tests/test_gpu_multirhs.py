@@ -236,3 +236,30 @@ def test_matvec_multi_matches_columnwise_oracle(k, fp32):
     for j in range(k):
         yo = oracle.matvec(mat, X[:, j])
         assert np.linalg.norm(Y[:, j] - yo) / np.linalg.norm(yo) <= tol, j
+
+
+@pytest.mark.parametrize("max_iter", [1, 2, 3, 4, 5, 199, 200, 201, 202, 203])
+def test_multi_columns_that_stop_at_every_parity(max_iter):
+    """x takes the multiples of p two iterations at a time: columns that converge in one, two and three
+    iterations (sums of so many eigenvectors of the Laplacian) beside one that runs to the limit, on both
+    sides of the residual replacement."""
+    n = 56
+    mat = W.poisson7(n)
+    g = np.arange(1, n + 1) * np.pi / (n + 1)
+    z, y, x = np.meshgrid(g, g, g, indexing="ij")
+    modes = [np.sin(a * x) * np.sin(a * y) * np.sin(a * z) for a in (1, 3, 7)]
+    cols = [sum(modes[:m]).reshape(-1) for m in (1, 2, 3)] + [W.uniform_vector(mat.n, seed=6)]
+    B = np.stack(cols, 1)
+    k = B.shape[1]
+    dm = api.DeviceMatrix(mat)
+    db, dx = api.DeviceBuffer.from_numpy(B.reshape(-1)), api.DeviceBuffer(mat.n * k)
+    res = dm.solve_multi(db, dx, k, _prm(tol=1e-9, precond=0, max_iter=max_iter))
+    X = dx.numpy().reshape(mat.n, k)
+    for j in range(k):
+        xo, st, I, R = oracle.solve(mat, np.ascontiguousarray(B[:, j]), precond=0, tol=1e-9, max_iter=max_iter)
+        assert (res["status"][j] != 0) == (st != 0), j
+        if j < 3:
+            assert res["iters"][j] == int(I[4]) == min(j + 1, max_iter), (j, res["iters"][j], I[4])
+        else:
+            assert res["iters"][j] == max_iter
+        assert np.linalg.norm(X[:, j] - xo) <= 1e-9 * np.linalg.norm(xo), j
