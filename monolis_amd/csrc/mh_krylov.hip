@@ -1415,9 +1415,22 @@ int cg_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& W, Sol
   // its own kernel and leaves (r, z) in parts_v.
   const bool vprec = PREC && B == 1 && M.vb != nullptr;
   const int ntile_v = vprec ? rows_grid<T, kVPrecBS>(M.vb->nb) : 0;
+  // blocks of up to kVPrecRegs rows: the update and diag_V are one kernel, which
+  // leaves (r, r) and (r, z) together (past the first and the replacement steps)
+  const bool vfused = vprec && M.vb->maxb <= kVPrecRegs;
+  const int nwg_vf = vfused ? (M.vb->nb + kVUpdBlocks - 1) / kVUpdBlocks : 0;
   auto upd = [&](int it, int flags) -> int {
     const double* pre = (flags & (F_UPD | F_XONLY)) ? parts_s : nullptr;
     if constexpr (PREC && B == 1) {
+      if (vfused && flags == F_UPD) {
+        const VBlock& V = *M.vb;
+        const T* DV = sizeof(T) == 8 ? (const T*)V.D64.p : (const T*)V.D32.p;
+        k_v_cg_update<T><<<nwg_vf, kBlock, 0, s>>>(V.nb, x, r, z, p, q, V.list.p, V.dof_index.p, V.doff.p, DV, st, it,
+                                                   pre, nwg_s, parts_u);
+        MH_HIP(hipGetLastError());
+        ktimer_mark(kClsPrec);
+        return 0;
+      }
       if (vprec) {
         OpCgUpdate<T, B, false> op{x, r, z, p, q, nullptr, n, st, it, flags | F_EXTPREC, pre, nwg_s, (T)0};
         MH_TRY((launch_rows<decltype(op), false>(n, op, parts_u, s)));
@@ -1432,6 +1445,8 @@ int cg_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& W, Sol
     return launch_rows<decltype(op), false>(n, op, parts_u, s);
   };
   auto p_op = [&](int it) {
+    if (vfused && it > 1 && (it - 1) % kIterRR != 0)
+      return OpCgP<T>{z, p, st, hp, parts_u, nwg_vf, nullptr, 0, it, (T)0};
     return OpCgP<T>{z, p, st, hp, parts_u, ntile_u, vprec ? parts_v : nullptr, ntile_v, it, (T)0};
   };
   MH_TRY(upd(0, 0));  // z = M^-1 r and the partials of the first rho

@@ -13,7 +13,7 @@ from monolis_amd import api
 from monolis_amd import matrix as mm
 from monolis_amd._lib import MonolisHipError
 
-from _helpers import random_bcsr, random_vblock
+from _helpers import _store_vblock_dense, random_bcsr, random_vblock
 from test_oracle_vblock import reference_matvec_v_case
 
 pytestmark = pytest.mark.gpu
@@ -177,3 +177,38 @@ def test_fixed_block_above_16_is_rejected():
     m = random_bcsr(10, 17, 0.3, seed=1, spd=True)
     with pytest.raises(MonolisHipError, match="16"):
         api.DeviceMatrix(m)
+
+
+# one block, a workgroup's 256 block rows less one and more one, two workgroups; blocks that the fused update
+# takes (up to 6 rows) and larger ones
+@pytest.mark.parametrize("n, maxb", [(1, 6), (255, 2), (257, 6), (600, 6), (257, 8)])
+def test_v_cg_update_sizes(n, maxb):
+    sizes = np.random.default_rng(n).integers(1, maxb + 1, n)
+    sizes[-1] = maxb
+    m = random_vblock(n, 0.01, 7, sizes=sizes)
+    b = np.random.default_rng(8).uniform(-1, 1, m.nndof)
+    dm = api.DeviceMatrix(m)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(m.npndof)
+    prm = api.Prm().quiet()
+    dm.solve(db, dx, prm)
+    xo, st, I, R = oracle.solve(m, b)
+    assert prm.Iarray[5] == 0 and st == 0 and _iter_ok(prm.Iarray[4], I[4])
+    assert np.linalg.norm(dx.numpy()[:m.nndof] - xo) <= 1e-6 * np.linalg.norm(xo)
+
+
+def test_v_cg_past_the_residual_replacement():
+    # a chain of 2,100 DOFs in blocks of 1, 2 and 3: more than 200 iterations
+    n = 1050
+    lst = np.array([1, 2, 3] * (n // 3), np.int32)
+    m = mm.nonzero_pattern_by_simple_mesh_V(n, lst, [(i, i + 1) for i in range(n - 1)])
+    N = int(lst.sum())
+    D = np.diag(np.full(N, 2.0 + 1e-3)) - np.diag(np.ones(N - 1), 1) - np.diag(np.ones(N - 1), -1)
+    _store_vblock_dense(m, D)
+    b = np.random.default_rng(9).uniform(-1, 1, N)
+    dm = api.DeviceMatrix(m)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(m.npndof)
+    prm = api.Prm().quiet()
+    dm.solve(db, dx, prm)
+    xo, st, I, R = oracle.solve(m, b)
+    assert prm.Iarray[5] == 0 and st == 0 and I[4] > 200 and _iter_ok(prm.Iarray[4], I[4]), (prm.Iarray[4], I[4])
+    assert np.linalg.norm(dx.numpy()[:N] - xo) <= 1e-6 * np.linalg.norm(xo)
