@@ -9,7 +9,7 @@
 //
 // Layout: a system-aligned SELL-64 -- every system starts on a fresh 64-row
 // slice, so a workgroup walks only its own slices.  Three persistent kernels:
-//  * k_resident (mh_resident.hpp): the vectors stay on chip; the default where it
+//  * k_res_cg (mh_resident.hpp): the vectors stay on chip; the default where it
 //    fits;
 //  * k_batch_cg: each workgroup takes systems wg, wg + G, ... (largest first) and
 //    runs the whole CG loop with workgroup barriers only;
@@ -882,8 +882,8 @@ int batch_solve(Batch& B, const BatchParams& P, const double* b, double* x, int 
   if (grid < 1) grid = 1;
   auto enqueue = [&]() -> int {
     if (cfg == kCfgResident) {
-      const ResArgs A{b, x, z, p, q, O, nullptr, P.max_iter, P.tol, P.init_x, P.precond, kIterRR};
-      return res_launch(B.res, false, B.slice_ptr.p, B.val.p, B.dinv.p, A, B.nsys, B.wait_s, s);
+      const ResArgs A{b, x, z, p, q, O, nullptr, P.max_iter, P.tol, P.init_x, P.precond};
+      return res_launch(B.res, B.slice_ptr.p, B.val.p, B.dinv.p, A, B.nsys, B.wait_s, s);
     }
     const int nctl = S ? 2 + S->nteam : 0;
     k_batch_reset<<<(std::max(B.nsys, nctl) + 255) / 256, 256, 0, s>>>(B.nsys, B.iters.p, B.resid.p, B.status.p,

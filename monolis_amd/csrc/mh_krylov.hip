@@ -1284,13 +1284,12 @@ size_t cg_bytes(const Matrix& M, int nvec, int max_iter) {
 }
 
 
-// The on-chip CG or BiCGSTAB on a scalar system (mh_resident.hpp): one launch
-// instead of three or five per iteration.  *ran stays false when the system does
-// not fit, when a team's wait gave up, or at an exact zero dot of BiCGSTAB (x is
-// then as it was); the launch-per-step solver follows, with its sorted-sum
-// fallback.  Solves with a time split take that one too: it times its steps.
-int solve_on_chip(Matrix& M, const SolveParams& P, bool bicgstab, int rr_period, bool prec, const double* b, double* x,
-                  Workspace& W, SolveResult* out, bool* ran, hipStream_t s) {
+// The on-chip CG on a scalar system (mh_resident.hpp): one launch instead of
+// three per iteration.  *ran stays false when the system does not fit, or when
+// a team's wait gave up (x is then as it was); the launch-per-step solver
+// follows.  Solves with a time split take that one too: it times its steps.
+int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, double* x, Workspace& W,
+               SolveResult* out, bool* ran, hipStream_t s) {
   *ran = false;
   if (M.n < 1 || M.n != M.np || P.max_iter < 1 || active_ktimer()) return 0;
   if ((long long)M.nslices > (long long)kResTeamMax * kResRowsLarge * kResNW) return 0;
@@ -1303,11 +1302,8 @@ int solve_on_chip(Matrix& M, const SolveParams& P, bool bicgstab, int rr_period,
                           M.col.p, nullptr, M.rowptr.p, cu_count(), s));
   }
   // With the matrix in registers always; otherwise while a member streams at
-  // most 300 KB per product (about 10 us from one CU).
-  const bool regs = bicgstab ? M.res->rp_bi == kResRowsMini : M.res->mr;
-  if (!M.res->fits || (bicgstab && M.res->rp_bi == 0) ||
-      (!regs && (double)M.nslots * kWave * 10.0 > 300e3 * M.res->nmem))
-    return 0;
+  // most 300 KB per iteration (about 10 us from one CU).
+  if (!M.res->fits || (!M.res->mr && (double)M.nslots * kWave * 10.0 > 300e3 * M.res->nmem)) return 0;
   struct Result {
     int iter, status;
     double resid;
@@ -1323,13 +1319,13 @@ int solve_on_chip(Matrix& M, const SolveParams& P, bool bicgstab, int rr_period,
   Result* d = cv.take<Result>(1);
   if (!P.init_x) MH_HIP(hipMemcpyAsync(x0, x, m * sizeof(double), hipMemcpyDeviceToDevice, s));
   const ResArgs a{b, x, z, p, xe, {&d->iter, &d->resid, &d->status}, P.keep_hist ? hist : nullptr, P.max_iter, P.tol,
-                  P.init_x, prec ? 1 : 0, rr_period};
-  MH_TRY(res_launch(*M.res, bicgstab, M.slice_ptr.p, M.val64.p, prec ? M.D64.p : nullptr, a, 1, 5.0, s));
+                  P.init_x, prec ? 1 : 0};
+  MH_TRY(res_launch(*M.res, M.slice_ptr.p, M.val64.p, prec ? M.D64.p : nullptr, a, 1, 5.0, s));
   MH_HIP(hipMemcpyAsync(&h, d, sizeof(Result), hipMemcpyDeviceToHost, s));
   MH_HIP(hipStreamSynchronize(s));
   if (h.status < 0 || h.status > 2) {
     int gave_up = 0;
-    if (h.status != 4) MH_TRY(res_aborted(*M.res, &gave_up, s));
+    MH_TRY(res_aborted(*M.res, &gave_up, s));
     if (!P.init_x) MH_HIP(hipMemcpyAsync(x, x0, m * sizeof(double), hipMemcpyDeviceToDevice, s));
     return 0;
   }
@@ -1355,7 +1351,7 @@ int cg_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& W, Sol
   if constexpr (B == 1 && sizeof(T) == 8) {
     if (!PREC || !M.vb) {
       bool ran = false;
-      MH_TRY(solve_on_chip(M, P, false, kIterRR, PREC, b, x, W, out, &ran, s));
+      MH_TRY(cg_on_chip(M, P, PREC, b, x, W, out, &ran, s));
       if (ran) return 0;
     }
   }
@@ -1982,13 +1978,6 @@ int bicgstab_impl(Matrix& M, const SolveParams& P, const T* b, T* x, Workspace& 
                   hipStream_t s, int rr_period) {
   Context* c = nullptr;
   MH_TRY(context(&c));
-  if constexpr (B == 1 && sizeof(T) == 8) {
-    if (!PREC || !M.vb) {
-      bool ran = false;
-      MH_TRY(solve_on_chip(M, P, true, rr_period, PREC, b, x, W, out, &ran, s));
-      if (ran) return 0;
-    }
-  }
   const size_t vec = (size_t)M.np * B;
   MH_TRY(W.ensure(cg_bytes<T>(M, 8, P.max_iter)));
   Carve cv{W.raw.p};

@@ -1,4 +1,4 @@
-// Plans and launches of the on-chip solvers (mh_resident.hpp).
+// Plans and launches of the on-chip CG (mh_resident.hpp).
 #include <algorithm>
 #include <cmath>
 #include <vector>
@@ -114,9 +114,9 @@ __global__ void k_res_reset(int nsys, int* iters, double* resid, int* status, in
   if (i < npart) part[i] = 0;  // no tag of an earlier launch
 }
 
-template <int RP, bool MR, bool BI>
+template <int RP, bool MR>
 int occupancy(size_t lds, int* per_cu) {
-  auto* k = &k_resident<RP, MR, BI>;
+  auto* k = &k_res_cg<RP, MR>;
   MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
   *per_cu = 0;
   MH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k, kResNT, lds));
@@ -241,20 +241,12 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
   plan.lds_bytes = (size_t)(plan.mr && !mini ? lds_mr : lds) * sizeof(double);
   int per_cu = 0;
   plan.rp = mini ? kResRowsMini : plan.mr || (small && plan.lds_bytes <= ((size_t)79 << 10)) ? kResRowsSmall : kResRowsLarge;
-  if (mini) MH_TRY((occupancy<kResRowsMini, true, false>(plan.lds_bytes, &per_cu)));
-  else if (plan.mr) MH_TRY((occupancy<kResRowsSmall, true, false>(plan.lds_bytes, &per_cu)));
-  else if (plan.rp == kResRowsSmall) MH_TRY((occupancy<kResRowsSmall, false, false>(plan.lds_bytes, &per_cu)));
-  else MH_TRY((occupancy<kResRowsLarge, false, false>(plan.lds_bytes, &per_cu)));
+  if (mini) MH_TRY((occupancy<kResRowsMini, true>(plan.lds_bytes, &per_cu)));
+  else if (plan.mr) MH_TRY((occupancy<kResRowsSmall, true>(plan.lds_bytes, &per_cu)));
+  else if (plan.rp == kResRowsSmall) MH_TRY((occupancy<kResRowsSmall, false>(plan.lds_bytes, &per_cu)));
+  else MH_TRY((occupancy<kResRowsLarge, false>(plan.lds_bytes, &per_cu)));
   if (per_cu < 1) return 0;
   plan.grid = std::min(plan.nmem, per_cu * cu_count());
-  // BiCGSTAB: six vectors in registers, with the matrix for four rows per thread, without for eight
-  plan.rp_bi = 0;
-  plan.lds_bi = (size_t)lds * sizeof(double);
-  if (small) {
-    if (mini) MH_TRY((occupancy<kResRowsMini, true, true>(plan.lds_bi, &per_cu)));
-    else MH_TRY((occupancy<kResRowsSmall, false, true>(plan.lds_bi, &per_cu)));
-    if (per_cu >= 1 && plan.nmem <= cu_count()) plan.rp_bi = mini ? kResRowsMini : kResRowsSmall;
-  }
   int dev = 0, khz = 0;
   MH_HIP(hipGetDevice(&dev));
   if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0) khz = 100000;
@@ -263,7 +255,7 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
   return 0;
 }
 
-int res_launch(const ResPlan& plan, bool bicgstab, const int* d_slice_ptr, const double* val, const double* dinv, const ResArgs& a,
+int res_launch(const ResPlan& plan, const int* d_slice_ptr, const double* val, const double* dinv, const ResArgs& a,
                int nsys, double wait_s, hipStream_t s) {
   const int npart = plan.nteam * 8 * kResTeamMax;
   k_res_reset<<<(std::max(nsys, npart + 2) + kBlock - 1) / kBlock, kBlock, 0, s>>>(
@@ -272,13 +264,10 @@ int res_launch(const ResPlan& plan, bool bicgstab, const int* d_slice_ptr, const
   const ResView V{plan.nmem, (const ResMember*)plan.mem.p, d_slice_ptr, plan.g_ptr.p, val, (const uint4*)plan.lcol.p,
                   plan.expf.p, dinv, plan.halo.p, plan.ctl.p, plan.part.p, (long long)(plan.ticks_per_s * wait_s),
                   plan.sticky.p};
-  if (bicgstab) {
-    if (plan.rp_bi == kResRowsMini) k_resident<kResRowsMini, true, true><<<plan.nmem, kResNT, plan.lds_bi, s>>>(V, a);
-    else k_resident<kResRowsSmall, false, true><<<plan.nmem, kResNT, plan.lds_bi, s>>>(V, a);
-  } else if (plan.rp == kResRowsMini) k_resident<kResRowsMini, true, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
-  else if (plan.mr) k_resident<kResRowsSmall, true, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
-  else if (plan.rp == kResRowsSmall) k_resident<kResRowsSmall, false, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
-  else k_resident<kResRowsLarge, false, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  if (plan.rp == kResRowsMini) k_res_cg<kResRowsMini, true><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  else if (plan.mr) k_res_cg<kResRowsSmall, true><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  else if (plan.rp == kResRowsSmall) k_res_cg<kResRowsSmall, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  else k_res_cg<kResRowsLarge, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
   MH_HIP(hipGetLastError());
   return 0;
 }

@@ -36,6 +36,7 @@ constexpr int kResNW = kResNT / kWave;
 constexpr int kResTeamMax = 128;            // workgroups per team at most (one wavefront polls 4 words of each)
 constexpr int kResLds = 20320;              // doubles of LDS for p (158.75 KB of the CU's 160)
 constexpr int kResSpinMax = 1 << 24;        // polls of one team wait at most (a bound that needs no clock)
+constexpr int kResIterRR = 200;             // residual replacement (CG.f90:91-95)
 constexpr int kResRowsLarge = 26;           // RP: 13,312 rows per member (150 VGPRs of vectors)
 constexpr int kResRowsMini = 4;             // RP: 2,048 rows
 constexpr int kResRowsSmall = 8;            // RP: 4,096 rows (with the matrix in registers: 208 VGPRs of data)
@@ -70,7 +71,7 @@ struct ResView {
 struct BatchOut {
   int* iters;
   double* resid;
-  int* status;   // 0 converged, 1 not converged, 2 zero rhs, 3 a team wait gave up, 4 an exact zero dot (BiCGSTAB)
+  int* status;   // 0 converged, 1 not converged, 2 zero rhs, 3 a team wait gave up
 };
 
 struct ResArgs {
@@ -84,7 +85,6 @@ struct ResArgs {
   int max_iter;
   double tol;
   int init_x, precond;
-  int rr_period;   // iterations between residual replacements
 };
 
 // Workgroup state beside the LDS vector.
@@ -123,9 +123,9 @@ __device__ __forceinline__ bool res_on(int left, int i) {
   return i * kResNW < left;
 }
 
-// One member's part of one system: CG, or BiCGSTAB (BI).
-template <int RP, bool W8, bool MR, bool BI>
-__device__ __forceinline__ void res_solve(const ResView& V, const ResMember& m, const ResArgs& a, double* lds,
+// One member's part of one system.
+template <int RP, bool W8, bool MR>
+__device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, const ResArgs& a, double* lds,
                                        ResShared& sh) {
   const int lane = threadIdx.x & (kWave - 1);
   const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x / kWave));
@@ -134,7 +134,7 @@ __device__ __forceinline__ void res_solve(const ResView& V, const ResMember& m, 
   // Row i of a thread: slice w + i*8 of the member, its lane.  With eight rows of
   // the matrix in registers x lies in LDS, behind p; with four the preconditioner
   // and the first halo rows' numbers are held in registers too.
-  constexpr bool XL = MR && RP > kResRowsMini, KEEP = (MR && RP <= kResRowsMini) || BI;
+  constexpr bool XL = MR && RP > kResRowsMini, KEEP = MR && RP <= kResRowsMini;
   constexpr int HU = 4;  // halo rows per thread and step
   double x[XL ? 1 : RP], r[RP], q[RP], dreg[KEEP ? RP : 1];
   int hreg[KEEP ? HU : 1];
@@ -388,105 +388,6 @@ __device__ __forceinline__ void res_solve(const ResView& V, const ResMember& m, 
   const bool init = a.init_x != 0;
   for_rows([&](int i, int l, bool, int g) { xv(i, l) = init ? 0.0 : a.x[g]; });
   load_vec([&](int i, int l, int) { return xv(i, l); }, init ? nullptr : a.x);
-  if constexpr (BI) {
-    // BiCGSTAB (BiCGSTAB.f90:80-175).  LDS holds the vector the next product
-    // takes: x (step 0: initial residual, replacement), pt = M^-1 p (1) or
-    // st = M^-1 s (2); pt and st are formed from p and s where they are used, s
-    // takes r's registers and t stays in q.  Five exchanges per iteration: three
-    // reductions, and one after each of the two input vectors is published.
-    double rt[RP], p[RP], v[RP];
-#pragma unroll
-    for (int i = 0; i < RP; ++i) rt[i] = p[i] = v[i] = 0.0;
-    int step = 0, it = 0;
-    double B2 = 0.0, rho = 0.0, alpha = 0.0, omega = 0.0, resid = 1.0;
-    auto broke = [&]() { finish(it, resid, 4); };
-    for (;;) {
-      product();
-      double d0 = 0.0, d1 = 0.0;
-      int next = -1;  // the next product's input, or -1: the end of an iteration
-      if (step == 0) {
-        for_rows([&](int i, int, bool real, int g) { r[i] = real ? a.b[g] - q[i] : 0.0; });
-      } else if (step == 1) {
-        for_rows([&](int i, int, bool, int) {
-          v[i] = q[i];
-          d0 = fma(rt[i], q[i], d0);
-        });
-        if (!sum(d0, d1)) return fail();
-        if (__builtin_amdgcn_readfirstlane(d0 == 0.0)) return broke();
-        alpha = rho / d0;
-        for_rows([&](int i, int, bool, int) { r[i] = fma(-alpha, v[i], r[i]); });  // s
-        next = 2;
-      } else {
-        for_rows([&](int i, int, bool, int) {
-          d0 = fma(q[i], r[i], d0);
-          d1 = fma(q[i], q[i], d1);
-        });
-        if (!sum(d0, d1)) return fail();
-        if (__builtin_amdgcn_readfirstlane(d1 == 0.0)) return broke();
-        omega = d0 / d1;
-        for_rows([&](int i, int, bool, int) {
-          x[i] = x[i] + alpha * (dreg[i] * p[i]) + omega * (dreg[i] * r[i]);
-          r[i] = fma(-omega, q[i], r[i]);
-        });
-        if (it % a.rr_period == 0) next = 0;
-      }
-      if (next < 0) {
-        d0 = d1 = 0.0;
-        for_rows([&](int i, int, bool, int) {
-          if (it == 0) rt[i] = r[i];
-          d0 = fma(r[i], r[i], d0);
-          d1 = fma(r[i], rt[i], d1);
-        });
-        if (!sum(d0, d1)) return fail();
-        double beta = 0.0;
-        if (it == 0) {
-          B2 = d0;
-          if (__builtin_amdgcn_readfirstlane(B2 == 0.0)) {  // mat_converge.f90:40-48
-            store_x(true);
-            return finish(0, 0.0, 2);
-          }
-          d1 = d0;  // RT == R
-        } else {
-          resid = sqrt(d0 / B2);
-          if (a.hist && m.rank == 0 && threadIdx.x == 0) a.hist[it] = resid;
-          const bool conv = __builtin_amdgcn_readfirstlane(resid < a.tol);
-          if (conv || it >= a.max_iter) {
-            store_x(false);
-            return finish(it, resid, conv ? 0 : 1);
-          }
-          if (__builtin_amdgcn_readfirstlane(d1 == 0.0)) return broke();
-          beta = (d1 / rho) * (alpha / omega);
-        }
-        rho = d1;
-        ++it;
-        for_rows([&](int i, int, bool, int) { p[i] = it > 1 ? r[i] + beta * (p[i] - omega * v[i]) : r[i]; });
-        next = 1;
-      }
-      step = next;
-      for_rows([&](int i, int l, bool real, int g) {
-        const double u = step == 1 ? dreg[i] * p[i] : step == 2 ? dreg[i] * r[i] : x[i];
-        lds[l] = u;
-        if ((exports >> i) & 1)
-          if (real) st_agent(a.z + g, u);
-      });
-      if (T > 1) {
-        double n0 = 0.0, n1 = 0.0;
-        if (!sum(n0, n1)) return fail();
-        for (int h0 = threadIdx.x; h0 < m.nhalo; h0 += HU * kResNT) {
-          double zv[HU];
-#pragma unroll
-          for (int u = 0; u < HU; ++u) {
-            const int h = h0 + u * kResNT;
-            zv[u] = ld_agent(a.z + (h0 < HU * kResNT ? hreg[u] : halo[h < m.nhalo ? h : 0]));
-          }
-#pragma unroll
-          for (int u = 0; u < HU; ++u)
-            if (h0 + u * kResNT < m.nhalo) lds[own + h0 + u * kResNT] = zv[u];
-        }
-      }
-      __syncthreads();
-    }
-  } else {
   // One loop body holds the only matrix product and the only preconditioner
   // pass.  LDS holds x when `resid_step` (the initial residual and the
   // replacement every 200 iterations), else p.
@@ -503,7 +404,7 @@ __device__ __forceinline__ void res_solve(const ResView& V, const ResMember& m, 
       alpha = rho / rr;  // (p, q)
       rr = 0.0;
       for_rows([&](int i, int l, bool, int) { xv(i, l) = fma(alpha, lds[l], xv(i, l)); });
-      if (it % a.rr_period == 0) {
+      if (it % kResIterRR == 0) {
         // the true residual: p is set aside while LDS holds x
         for_rows([&](int i, int l, bool real, int g) {
           if (real) {
@@ -579,16 +480,15 @@ __device__ __forceinline__ void res_solve(const ResView& V, const ResMember& m, 
     for_rows([&](int i, int l, bool, int) { lds[l] = fma(beta, lds[l], q[i]); });
     __syncthreads();
   }
-  }
 }
 
 // Persistent: workgroups take members in order from one counter.  A team's
 // members are consecutive, so at most one team is incomplete at any time and a
 // member waiting for a teammate that has not started waits only for running
 // workgroups to finish their own complete teams.
-template <int RP, bool MR, bool BI>
-__global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP <= kResRowsSmall && !MR && !BI ? 4 : 2)))
-    k_resident(ResView V, ResArgs a) {
+template <int RP, bool MR>
+__global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP <= kResRowsSmall && !MR ? 4 : 2)))
+    k_res_cg(ResView V, ResArgs a) {
   extern __shared__ double res_lds[];
   __shared__ ResShared sh;
   for (;;) {
@@ -598,10 +498,10 @@ __global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP 
     if (k >= V.nmem) break;
     const ResMember m = V.mem[k];
     if constexpr (MR) {
-      res_solve<RP, true, true, BI>(V, m, a, res_lds, sh);
+      res_cg<RP, true, true>(V, m, a, res_lds, sh);
     } else {
-      if (m.w8) res_solve<RP, true, false, BI>(V, m, a, res_lds, sh);
-      else res_solve<RP, false, false, BI>(V, m, a, res_lds, sh);
+      if (m.w8) res_cg<RP, true, false>(V, m, a, res_lds, sh);
+      else res_cg<RP, false, false>(V, m, a, res_lds, sh);
     }
     __syncthreads();
   }
@@ -617,9 +517,7 @@ struct ResSystem {
 struct ResPlan {
   bool fits = false;
   int nmem = 0, nteam = 0, grid = 0, rp = 0;
-  bool mr = false;  // CG: the members' matrix stays in registers
-  int rp_bi = 0;    // rows per thread for BiCGSTAB: 4 (matrix in registers), 8, or 0 (does not fit)
-  size_t lds_bi = 0;
+  bool mr = false;  // the members' matrix stays in registers
   size_t lds_bytes = 0;
   double ticks_per_s = 0;
   DevArray<unsigned char> mem, expf, lcol;
@@ -634,9 +532,8 @@ struct ResPlan {
 int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
                    const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int team_limit,
                    hipStream_t s);
-// Zeroes the counters and enqueues the solver (both capturable); BiCGSTAB only
-// when plan.rp_bi is set.
-int res_launch(const ResPlan& plan, bool bicgstab, const int* d_slice_ptr, const double* val, const double* dinv, const ResArgs& a,
+// Zeroes the counters and enqueues the solver (both capturable).
+int res_launch(const ResPlan& plan, const int* d_slice_ptr, const double* val, const double* dinv, const ResArgs& a,
                int nsys, double wait_s, hipStream_t s);
 // 1 when a team wait gave up in any launch since the last call (synchronises).
 int res_aborted(ResPlan& plan, int* aborted, hipStream_t s);
