@@ -81,17 +81,39 @@ __device__ __forceinline__ double read_lane(double v, int lane) {
   return __longlong_as_double((long long)hi << 32 | (unsigned)lo);
 }
 
-// Sum over the wavefront, in every lane.  Rows of 16 by four DPP moves (lanes
-// 1, 2, 7 - i and 15 - i away), then the four row sums through scalar registers:
-// no LDS round trip, where six shuffles were 12 dependent LDS permutes (the
-// on-chip CG on 10^3 rows: 5.1 -> 4.0 us per iteration with two pairs of sums).
-// All 64 lanes must be active.
+// v of the lane 32 (16) away plus the lane's own: v_permlane32_swap (16) of two
+// copies leaves each half's (row's) value in both.
+template <int O>
+__device__ __forceinline__ double swap_add(double v) {
+  static_assert(O == 32 || O == 16, "halves or rows");
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)b, hi = (unsigned)(b >> 32);
+  unsigned l0, l1, h0, h1;
+  if constexpr (O == 32) {
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+  } else {
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    l0 = l[0], l1 = l[1], h0 = h[0], h1 = h[1];
+  }
+  return __longlong_as_double((long long)h0 << 32 | l0) + __longlong_as_double((long long)h1 << 32 | l1);
+}
+
+// Sum over the wavefront, in every lane: the butterfly over lanes 32, 16, 8, 4, 2
+// and 1 away, by lane swaps and DPP moves.  The same tree as six shuffles, so the
+// same bits, without their 12 dependent LDS permutes (the on-chip CG on 10^3
+// rows, two pairs of sums per iteration: 5.1 -> 4.0 us).  All 64 lanes must be
+// active.
 __device__ __forceinline__ double wave_sum(double v) {
-  v += dpp_move<0xB1>(v);   // quad_perm 1,0,3,2
-  v += dpp_move<0x4E>(v);   // quad_perm 2,3,0,1
-  v += dpp_move<0x141>(v);  // row_half_mirror
-  v += dpp_move<0x140>(v);  // row_mirror
-  return (read_lane(v, 0) + read_lane(v, 16)) + (read_lane(v, 32) + read_lane(v, 48));
+  v = swap_add<32>(v);
+  v = swap_add<16>(v);
+  v += dpp_move<0x128>(v);                   // row_ror 8: lane ^ 8
+  v += dpp_move<0x1B>(dpp_move<0x141>(v));   // row_half_mirror, quad_perm 3,2,1,0: lane ^ 4
+  v += dpp_move<0x4E>(v);                    // quad_perm 2,3,0,1: lane ^ 2
+  v += dpp_move<0xB1>(v);                    // quad_perm 1,0,3,2: lane ^ 1
+  return v;
 }
 
 __device__ __forceinline__ int wave_max(int v) {

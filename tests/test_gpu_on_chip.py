@@ -1,0 +1,128 @@
+"""Scalar CG solves that run in one launch with the vectors on chip,
+against the launch-per-step solver on the same handle (taken by a solve with the
+time split on) and the oracle: same status, iteration counts within +-2 % (+-1 below
+50), solutions within 1e-6."""
+import numpy as np
+import pytest
+
+import oracle
+from monolis_amd import api, workloads as W
+from monolis_amd.matrix import Matrix
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _init(hip):
+    oracle.set_threads(1)
+    yield
+
+
+def _matrix(n, far, wide, seed):
+    """Diagonally dominant rows of uneven length (1 entry in every fifth row, more than 8 with `wide`),
+    some coupling `far` rows apart."""
+    rng = np.random.default_rng(seed)
+    reps = 4 if wide else 1
+    i = rng.integers(0, n, reps * n)
+    d = np.where(rng.uniform(size=reps * n) < 0.3, far, rng.integers(1, 30, reps * n))
+    keep = (i + d < n) & (i % 5 != 0) & ((i + d) % 5 != 0)
+    if not wide:   # at most 3 entries on each side of the diagonal
+        _, first = np.unique(i, return_index=True)
+        one = np.zeros(reps * n, bool)
+        one[first] = True
+        keep &= one & (rng.uniform(size=reps * n) < 0.9)
+    key = np.unique(i[keep] * n + i[keep] + d[keep])
+    i, j = key // n, key % n
+    v = -rng.uniform(0.1, 1.0, len(i))
+    rows, cols = np.concatenate([i, j, np.arange(n)]), np.concatenate([j, i, np.arange(n)])
+    off = np.bincount(np.concatenate([i, j]), weights=np.abs(np.concatenate([v, v])), minlength=n)
+    vals = np.concatenate([v, v, off + 0.05])
+    order = np.lexsort((cols, rows))
+    index = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    return Matrix(n, n, 1, index, (cols[order] + 1).astype(np.int32), vals[order]).ensure_dof_index()
+
+
+def _prm(precond=1, tol=1e-8, steps=False, init_x=True, max_iter=3000):
+    prm = api.Prm().quiet()
+    prm.Iarray[api.MONOLIS_PRM_I_PRECOND] = precond
+    prm.Iarray[api.MONOLIS_PRM_I_MAX_ITER] = max_iter
+    prm.Iarray[api.MONOLIS_PRM_I_IS_MEASUREMENT] = int(steps)
+    prm.Iarray[api.MONOLIS_PRM_I_IS_INIT_X] = int(init_x)
+    prm.Rarray[api.MONOLIS_PRM_R_TOL] = tol
+    return prm
+
+
+def _near(a, b):
+    return abs(a - b) <= max(1, int(0.02 * max(a, b)))
+
+
+def _both(mat, b, precond=1, x0=None, **kw):
+    """(x, iterations, residual history) on chip and step by step."""
+    dm = api.DeviceMatrix(mat)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
+    out = []
+    for steps in (False, True):
+        if x0 is not None:
+            dx.upload(x0)
+        prm = _prm(precond, steps=steps, init_x=x0 is None, **kw)
+        h = dm.solve(db, dx, prm, hist_len=3001)
+        it = int(prm.Iarray[api.MONOLIS_PRM_I_CUR_ITER])
+        out.append((dx.numpy(), it, h, int(prm.Iarray[api.MONOLIS_PRM_I_IERR]), prm.Rarray[api.MONOLIS_PRM_R_CUR_RESID]))
+    (x, it, h, st, res), (xs, its, hs, sts, ress) = out
+    assert st == sts and _near(it, its), (it, its)
+    assert np.linalg.norm(x - xs) <= 1e-6 * np.linalg.norm(xs)
+    assert h[it] == res and np.all(h[1:it + 1] >= 0) and not h[it + 1:].any()
+    k = min(5, it, its)
+    assert np.allclose(h[1:k], hs[1:k], rtol=1e-6)
+    return x, it
+
+
+# one row, a whole and a partial slice, one member and the first team, four and eight rows per thread, rows
+# of more and fewer than eight entries
+@pytest.mark.parametrize("precond", [1, 0])
+@pytest.mark.parametrize("n, far, wide", [(1, 1, False), (64, 5, False), (1000, 333, True), (2048, 700, False),
+                                          (2049, 700, True), (70001, 9000, False), (70001, 2000, True)])
+def test_on_chip_matches_steps_and_oracle(n, far, wide, precond):
+    mat = _matrix(n, far, wide, seed=n + wide)
+    b = oracle.matvec(mat, W.uniform_vector(n, seed=2))
+    x, it = _both(mat, b, precond)
+    xo, st, I, R = oracle.solve(mat, b, precond=precond, max_iter=3000)
+    assert st == 0 and _near(it, int(I[4]))
+    assert np.linalg.norm(x - xo) <= 1e-6 * np.linalg.norm(xo)
+
+
+def test_on_chip_past_the_replacement_and_from_a_start_vector():
+    # 64^3 rows take the largest team four rows per thread, 72^3 eight, with x in LDS
+    for e in (64, 72):
+        mat = W.poisson7(e)
+        b = W.uniform_vector(mat.n, seed=3)
+        x, it = _both(mat, b, tol=1e-11)
+        assert it > 200
+        # both end within tol * ||r0|| * cond of the solution: 1.8e-6 apart at 1e-8 from this start, 1e-8 here
+        _both(mat, b, x0=W.uniform_vector(mat.n, seed=4), tol=1e-10)
+
+
+def test_on_chip_zero_rhs_limit_and_repeat():
+    mat = _matrix(5000, 600, False, 9)
+    dm = api.DeviceMatrix(mat)
+    db, dx = api.DeviceBuffer.from_numpy(np.zeros(5000)), api.DeviceBuffer.from_numpy(np.ones(5000))
+    dm.solve(db, dx, _prm())
+    assert not dx.numpy().any()
+    b = W.uniform_vector(5000, seed=1)
+    db.upload(b)
+    prm = _prm(max_iter=7)
+    dm.solve(db, dx, prm)
+    assert prm.Iarray[api.MONOLIS_PRM_I_IERR] == 1 and prm.Iarray[api.MONOLIS_PRM_I_CUR_ITER] == 7
+    xo, st, I, R = oracle.solve(mat, b, max_iter=7)
+    assert np.linalg.norm(dx.numpy() - xo) <= 1e-6 * np.linalg.norm(xo)
+    dm.solve(db, dx, _prm())
+    x = dx.numpy()
+    for _ in range(3):
+        dm.solve(db, dx, _prm())
+        assert np.array_equal(x, dx.numpy())
+    # new values on the same pattern
+    dm.set_values(mat.A * 2.0)
+    dm.solve(db, dx, _prm())
+    mat2 = Matrix(5000, 5000, 1, mat.index, mat.item, mat.A * 2.0).ensure_dof_index()
+    xo, st, I, R = oracle.solve(mat2, b)
+    assert np.linalg.norm(dx.numpy() - xo) <= 1e-6 * np.linalg.norm(xo)
