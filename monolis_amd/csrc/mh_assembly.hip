@@ -468,26 +468,33 @@ __device__ __forceinline__ zd bc_prod(zd v, zd a) {
   return zd(v.re * a.re - v.im * a.im, v.re * a.im + v.im * a.re);
 }
 
-// One thread per block row: rows of condition DOFs become unit rows with
-// rhs = val; other rows move val * A(r, c) of condition columns to the
-// right-hand side (blocks in column order, then component order) and zero them.
-// nodebc flags the nodes with a condition: most rows couple to none and end
-// after one pass over their column ids (134 -> 102 us for 12,675 conditions on
-// 274,625 rows of 27 blocks).
+// A workgroup per slice, one thread per block row: rows of condition DOFs become
+// unit rows with rhs = val; other rows move val * A(r, c) of condition columns to
+// the right-hand side (blocks in column order, then component order) and zero
+// them.  nodebc flags the nodes with a condition: the four wavefronts look over a
+// slice's column ids together, and most rows, coupling to none, end there (12,675
+// conditions on 274,625 rows of 27 blocks: 134 -> 83 us).
 template <typename V>
-__global__ void k_bc_apply(int n, int b, const int* __restrict__ slice_ptr, const int* __restrict__ rowptr,
-                           const int* __restrict__ col, V* __restrict__ val, const int* __restrict__ isbc,
-                           const int* __restrict__ nodebc, const V* __restrict__ bcval, V* __restrict__ rhs) {
+__global__ void __launch_bounds__(kBlock) k_bc_apply(int n, int b, const int* __restrict__ slice_ptr,
+                                                     const int* __restrict__ rowptr, const int* __restrict__ col,
+                                                     V* __restrict__ val, const int* __restrict__ isbc,
+                                                     const int* __restrict__ nodebc, const V* __restrict__ bcval,
+                                                     V* __restrict__ rhs) {
 #pragma clang fp contract(off)
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= n) return;
-  const int s = r / kWave, lane = r % kWave;
+  __shared__ int flag[kWpb][kWave];
+  const int s = blockIdx.x, lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+  const int r = s * kWave + lane;
   const int k0 = slice_ptr[s];
-  const int len = rowptr[r + 1] - rowptr[r];
+  const int len = r < n ? rowptr[r + 1] - rowptr[r] : 0;
   const int bb = b * b;
-  int any = nodebc[r];
-#pragma unroll 8
-  for (int k = 0; k < len; ++k) any |= nodebc[col[((size_t)k0 + k) * kWave + lane]];
+  int any = r < n ? nodebc[r] : 0;
+#pragma unroll 4
+  for (int k = w; k < len; k += kWpb) any |= nodebc[col[((size_t)k0 + k) * kWave + lane]];
+  flag[w][lane] = any;
+  __syncthreads();
+  if (w != 0) return;
+#pragma unroll
+  for (int u = 1; u < kWpb; ++u) any |= flag[u][lane];
   if (!any) return;
   for (int k1 = 0; k1 < b; ++k1) {
     const bool rowbc = isbc[r * b + k1] != 0;
@@ -1113,7 +1120,7 @@ static int dirichlet_T(Matrix* M, V* rhs, int n_bc, const int* node, const int* 
     MH_TRY(upload(rtmp.p, rhs, m * sizeof(V), s));
     dr = rtmp.p;
   }
-  k_bc_apply<V><<<grid_for(M->n), kBlock, 0, s>>>(M->n, b, M->slice_ptr.p, M->rowptr.p, M->col.p, values_of<V>(M),
+  k_bc_apply<V><<<(M->n + kWave - 1) / kWave, kBlock, 0, s>>>(M->n, b, M->slice_ptr.p, M->rowptr.p, M->col.p, values_of<V>(M),
                                                   isbc.p, nodebc, bcval.p, dr);
   MH_HIP(hipGetLastError());
   if (!rhs_dev) MH_HIP(hipMemcpyAsync(rhs, dr, m * sizeof(V), hipMemcpyDeviceToHost, s));

@@ -379,25 +379,35 @@ int launch_sell_gather(const Matrix& M, const zd* val, zd* A, hipStream_t s) {
   return launch_sell_tile<zd, false>(M, A, val, nullptr, 0, s);
 }
 
-// Largest |col - row| over the stored slots of the valid rows (atomicMax).
-__global__ void k_col_span(int n, int nslices, const int* __restrict__ rowptr, const int* __restrict__ slice_ptr,
-                           const int* __restrict__ col, int* __restrict__ span) {
-  const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= (long long)nslices * kWave) return;
-  const int s = (int)(t / kWave), lane = (int)(t % kWave), row = (int)t;
+// Largest |col - row| over the stored slots of the valid rows.  Atomics on the
+// one address cost about 12 ns each (274,625 rows of 27 blocks: 54 us with one
+// per slice, 124 us with one per wavefront of a slice), so at most 512 workgroups
+// walk the slices, their wavefronts taking every fourth slot, with one atomic each
+// (19 us).
+constexpr int kSpanGrid = 512;
+__global__ void __launch_bounds__(kBlock) k_col_span(int n, int nslices, const int* __restrict__ rowptr,
+                                                     const int* __restrict__ slice_ptr, const int* __restrict__ col,
+                                                     int* __restrict__ span) {
+  __shared__ int top[kWpb];
+  const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
   int m = 0;
-  if (row < n) {
+  for (int s = blockIdx.x; s < nslices; s += gridDim.x) {
+    const int row = s * kWave + lane;
     const int k0 = slice_ptr[s];
-    const int len = rowptr[row + 1] - rowptr[row];
+    const int len = row < n ? rowptr[row + 1] - rowptr[row] : 0;
 #pragma unroll 4
-    for (int k = 0; k < len; ++k) {
+    for (int k = w; k < len; k += kWpb) {
       const int d = col[((size_t)k0 + k) * kWave + lane] - row;
       m = max(m, d < 0 ? -d : d);
     }
   }
-  // one atomic per wavefront (54 us on 274,625 rows of 27 blocks; 62 us with one per row)
   m = wave_max(m);
-  if (lane == 0 && m > 0) atomicMax(span, m);
+  if (lane == 0) top[w] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    for (int u = 1; u < kWpb; ++u) m = max(m, top[u]);
+    if (m > 0) atomicMax(span, m);
+  }
 }
 
 // 16-bit delta copy of the column ids: slot t of lane l goes to half (t & 1)
@@ -513,7 +523,8 @@ static int build_col16(Matrix* M, hipStream_t s) {
   MH_HIP(hipMemsetAsync(span.p, 0, sizeof(int), s));
   const long long threads = (long long)M->nslices * kWave;
   const unsigned grid = (unsigned)((threads + kBlock - 1) / kBlock);
-  k_col_span<<<grid, kBlock, 0, s>>>(M->n, M->nslices, M->rowptr.p, M->slice_ptr.p, M->col.p, span.p);
+  k_col_span<<<std::min(M->nslices, kSpanGrid), kBlock, 0, s>>>(M->n, M->nslices, M->rowptr.p, M->slice_ptr.p, M->col.p,
+                                                               span.p);
   MH_HIP(hipGetLastError());
   int h = 0;
   MH_HIP(hipMemcpyAsync(&h, span.p, sizeof(int), hipMemcpyDeviceToHost, s));
