@@ -591,7 +591,7 @@ __global__ void k_batch_fill(int nsys_rows_total, const int* __restrict__ sell_s
   }
 
 // Configuration 15: the on-chip CG (mh_resident.hpp).  512 Poisson systems of
-// 10^3..40^3 rows: 19.0 ms against 51.1 for the best of the others (the
+// 10^3..40^3 rows: 17.6 ms against 51.1 for the best of the others (the
 // vectors' 108 of 190 bytes per row and iteration stay on chip).  It is the
 // default of every batch it fits; one with a system it does not fit runs
 // kCfgFallback instead (also when configuration 15 is asked for).

@@ -7,7 +7,7 @@
 // then streams only the matrix -- 8 bytes of value and 2 bytes of LDS index per
 // entry -- and the preconditioner's 8 bytes per row: about 80 bytes per row of a
 // 7-point system against 190 with the vectors in memory.  512 Poisson systems of
-// 10^3..40^3 rows: 51.1 -> 19.0 ms, 1.377e9 row-iterations at 72 G/s (5.8 TB/s of
+// 10^3..40^3 rows: 51.1 -> 17.6 ms, 1.377e9 row-iterations at 78 G/s (6.3 TB/s of
 // those bytes): bound by the matrix stream.  A single 32^3 system: 1.93 -> 0.77
 // ms (17.7 -> 7.0 us per iteration, three launches before): bound by the two
 // exchanges and the halo loads, about 1 us each, and the sums' serial chains.
