@@ -198,9 +198,13 @@ int monolis_hip_matrix_autotune(monolis_hip_matrix* M, int fp32, int reps, int* 
  * solves of exactly `iters` iterations of `method` / `precond` (tolerance 0)
  * per SpMV variant in one precision (fp32 = 0 or 1, the FP32 copy that the
  * refined solve's inner iterations use) and keeps the fastest on the handle;
- * ms (if not NULL) gets monolis_hip_num_variants() milliseconds per iteration. */
+ * ms (if not NULL) gets monolis_hip_num_variants() milliseconds per iteration.
+ * The timed solves take the launch-per-step solver, whose SpMV the variant is. */
 int monolis_hip_matrix_autotune_solver(monolis_hip_matrix* M, int fp32, int method, int precond, int iters,
                                        int reps, int* best, double* ms);
+/* Solves of the handle so far that ran in one launch with the vectors on chip
+ * (FP64 CG on scalar systems that fit; the SpMV variant plays no part there). */
+int monolis_hip_matrix_on_chip_solves(const monolis_hip_matrix* M, int* solves);
 /* Forces a variant for one precision (fp32 = 0 or 1); an untuned handle uses
  * variant 4 (one wavefront per slice, 3 slots per step). */
 int monolis_hip_matrix_set_variant(monolis_hip_matrix* M, int fp32, int variant);

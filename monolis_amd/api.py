@@ -432,6 +432,13 @@ class DeviceMatrix:
                    "autotune_solver")
         return {"best": best.value, "ms_per_iter": list(ms)}
 
+    def on_chip_solves(self) -> int:
+        """Solves of this handle so far that ran in one launch with the vectors on chip."""
+        n = ctypes.c_int()
+        _lib.check(_lib.load().monolis_hip_matrix_on_chip_solves(ctypes.c_void_p(self.h), ctypes.byref(n)),
+                   "on_chip_solves")
+        return n.value
+
     def set_variant(self, variant: int, fp32: bool = False) -> None:
         _lib.check(_lib.load().monolis_hip_matrix_set_variant(ctypes.c_void_p(self.h), int(fp32), int(variant)),
                    "set_variant")

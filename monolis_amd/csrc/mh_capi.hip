@@ -795,10 +795,20 @@ int monolis_hip_matrix_autotune_solver(monolis_hip_matrix* H, int fp32, int meth
   P.tol = 0.0;
   P.keep_hist = 0;
   P.rhs_nonzero = 1;
+  P.steps = 1;  // the on-chip CG has no SpMV launch: every variant would time the same kernel
   Matrix& M = *H->M;
   if (fp32) rc = autotune_solver_T<float>(M, H->W, P, reps, best, ms, c->stream);
   else rc = autotune_solver_T<double>(M, H->W, P, reps, best, ms, c->stream);
   return rc ? (rc == -3 ? ST_PRECOND : rc == -4 ? ST_METHOD : rc == -2 ? ST_ARGS : ST_HIP) : 0;
+}
+
+int monolis_hip_matrix_on_chip_solves(const monolis_hip_matrix* H, int* solves) {
+  if (!H || !H->M || !solves) {
+    mh::set_error("on_chip_solves: null argument");
+    return ST_ARGS;
+  }
+  *solves = H->M->on_chip_solves;
+  return 0;
 }
 
 static mh::BatchParams batch_params(const int* Iarray, const double* Rarray) {

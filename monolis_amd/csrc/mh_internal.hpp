@@ -156,6 +156,7 @@ struct Matrix {
   bool transpose_stale = false;   // values of A changed since the transpose was filled
   VBlock* vb = nullptr;           // non-null for variable block sizes
   ResPlan* res = nullptr;         // built by the first solve that may run on chip
+  int on_chip_solves = 0;         // solves that ran on chip
   // complex matrices (monolis's *_C path): values in valz instead of val64,
   // complex block-Jacobi factors in Dz (same structure-of-arrays layout as D64)
   bool is_complex = false;
@@ -241,6 +242,7 @@ struct SolveParams {
   int chunk = 8;         // iterations enqueued between convergence polls
   int keep_hist = 1;     // record per-iteration residuals
   int rhs_nonzero = 0;   // caller guarantees b - A x0 != 0: skip the zero right-hand-side read-back
+  int steps = 0;         // launch-per-step solvers only (the SpMV variant tuning times their launches)
 };
 
 struct SolveResult {

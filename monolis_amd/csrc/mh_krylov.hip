@@ -1291,7 +1291,7 @@ size_t cg_bytes(const Matrix& M, int nvec, int max_iter) {
 int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, double* x, Workspace& W,
                SolveResult* out, bool* ran, hipStream_t s) {
   *ran = false;
-  if (M.n < 1 || M.n != M.np || P.max_iter < 1 || active_ktimer()) return 0;
+  if (M.n < 1 || M.n != M.np || P.max_iter < 1 || P.steps || active_ktimer()) return 0;
   if ((long long)M.nslices > (long long)kResTeamMax * kResRowsLarge * kResNW) return 0;
   if (!M.res) {
     M.res = new ResPlan();
@@ -1340,6 +1340,7 @@ int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, doub
     MH_HIP(hipMemcpyAsync(out->hist.data() + 1, hist + 1, sizeof(double) * (size_t)out->iter, hipMemcpyDeviceToHost, s));
     MH_HIP(hipStreamSynchronize(s));
   }
+  ++M.on_chip_solves;
   *ran = true;
   return 0;
 }

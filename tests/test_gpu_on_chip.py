@@ -126,3 +126,17 @@ def test_on_chip_zero_rhs_limit_and_repeat():
     mat2 = Matrix(5000, 5000, 1, mat.index, mat.item, mat.A * 2.0).ensure_dof_index()
     xo, st, I, R = oracle.solve(mat2, b)
     assert np.linalg.norm(dx.numpy() - xo) <= 1e-6 * np.linalg.norm(xo)
+
+
+def test_solver_tuning_times_the_launches_that_the_variant_is_of():
+    """The SpMV variants are those of the launch-per-step solver: tuning on a system that also fits on chip
+    takes that solver, with the unpreconditioned form as well; later solves run on chip again."""
+    mat = _matrix(3000, 500, False, 12)
+    dm = api.DeviceMatrix(mat)
+    for precond in (1, 0):
+        t = dm.autotune_solver(fp32=False, precond=precond, iters=6, reps=1)
+        assert dm.on_chip_solves() == 0
+        assert all(v > 0 for v in t["ms_per_iter"]) and t["ms_per_iter"][t["best"]] == min(t["ms_per_iter"])
+    db, dx = api.DeviceBuffer.from_numpy(W.uniform_vector(3000, seed=1)), api.DeviceBuffer(3000)
+    dm.solve(db, dx, _prm())
+    assert dm.on_chip_solves() == 1
