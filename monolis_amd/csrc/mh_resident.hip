@@ -114,10 +114,17 @@ __global__ void k_res_reset(int nsys, int* iters, double* resid, int* status, in
   if (i < npart) part[i] = 0;  // no tag of an earlier launch
 }
 
+// LDS of k_res_build's bitmap and its prefix (491,520 rows).
+constexpr size_t kResBuildLds = (size_t)120 << 10;
+
+// The attribute belongs to the kernel, which all plans of the process share: it
+// is set to the most that any of them takes, never to one plan's own size (a
+// smaller plan would lower it below what an earlier one launches with).
 template <int RP, bool MR>
 int occupancy(size_t lds, int* per_cu) {
   auto* k = &k_res_cg<RP, MR>;
-  MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+  MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
+                             (int)(kResLds * sizeof(double))));
   *per_cu = 0;
   MH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k, kResNT, lds));
   return 0;
@@ -136,7 +143,7 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
     maxrows = std::max(maxrows, q.rows);
   }
   const size_t build_lds = (size_t)((maxrows + 31) / 32) * 2 * sizeof(unsigned);
-  if (maxrows > kResTeamMax * kResRowsLarge * kResNT || build_lds > ((size_t)120 << 10)) return 0;
+  if (maxrows > kResTeamMax * kResRowsLarge * kResNT || build_lds > kResBuildLds) return 0;
   struct Task {
     int sys, T;
     double d;
@@ -215,7 +222,7 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
   MH_HIP(hipMemsetAsync(plan.expf.p, 0, (size_t)nslices, s));
   MH_HIP(hipMemsetAsync(plan.sticky.p, 0, 2 * sizeof(int), s));
   MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_res_build), hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)build_lds));
+                             (int)kResBuildLds));
   k_res_build<<<plan.nmem, kResNT, build_lds, s>>>((ResMember*)plan.mem.p, d_slice_ptr, plan.g_ptr.p, d_col, rowlen,
                                                    rowptr, plan.expf.p, plan.halo.p, (uint4*)plan.lcol.p,
                                                    plan.sticky.p + 1);

@@ -140,3 +140,36 @@ def test_solver_tuning_times_the_launches_that_the_variant_is_of():
     db, dx = api.DeviceBuffer.from_numpy(W.uniform_vector(3000, seed=1)), api.DeviceBuffer(3000)
     dm.solve(db, dx, _prm())
     assert dm.on_chip_solves() == 1
+
+
+def test_on_chip_handles_of_one_kernel_and_different_lds():
+    """Kernels are shared by the handles: an older handle that takes much LDS (members with a long halo) is
+    solved again after a younger one with little has been built, singly and as a batch."""
+    def handle(mat):
+        db, dx = api.DeviceBuffer.from_numpy(W.uniform_vector(mat.n, seed=5)), api.DeviceBuffer(mat.n)
+        return api.DeviceMatrix(mat), db, dx
+
+    # four rows per thread with the matrix in registers; eight; 26 rows per thread
+    for big, small in ((_matrix(70001, 9000, False, 1), _matrix(64, 5, False, 2)),
+                       (W.poisson7(72), W.poisson7(65)),
+                       (_matrix(70001, 9000, True, 1), _matrix(2049, 9, True, 2))):
+        a, b = handle(big), handle(small)
+        a[0].solve(a[1], a[2], _prm())
+        x = a[2].numpy()
+        b[0].solve(b[1], b[2], _prm())
+        a[2].upload(np.zeros(big.n))
+        a[0].solve(a[1], a[2], _prm())
+        assert a[0].on_chip_solves() == 2 and b[0].on_chip_solves() == 1
+        assert np.array_equal(x, a[2].numpy())
+    out = []
+    for edges in ([40, 40, 38], [8, 9]):
+        mat, sys_row = W.poisson_batch(edges=edges)
+        B = api.DeviceBatch(mat, sys_row)
+        assert B.schedule(15)["split"] == 1
+        db, dx = api.DeviceBuffer.from_numpy(W.uniform_vector(mat.n, seed=6)), api.DeviceBuffer(mat.n)
+        B.solve(db, dx, _prm())
+        out.append((B, db, dx, dx.numpy()))
+    B, db, dx, x = out[0]
+    dx.upload(np.zeros(len(x)))
+    B.solve(db, dx, _prm())
+    assert np.array_equal(x, dx.numpy())
