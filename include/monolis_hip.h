@@ -244,7 +244,10 @@ int monolis_hip_batch_set_config(monolis_hip_batch* B, int cfg);
  * task) and teams its schedule for B has. */
 int monolis_hip_batch_schedule(monolis_hip_batch* B, int cfg, int* split, int* nslot, int* nteam);
 /* Longest time in seconds (default 5, at most 600) that one team barrier waits
- * for a member before the launch gives up on the system (status 3). */
+ * for a member before the launch gives up on the system (status 3, and the call
+ * returns an error).  Configuration 15 redoes the batch without teams instead,
+ * from the same start vector, and so the following solves, until this limit or
+ * the configuration is set again; with limit 0 its teams give up at once. */
 int monolis_hip_batch_set_wait_limit(monolis_hip_batch* B, double seconds);
 int monolis_hip_batch_autotune(monolis_hip_batch* B, const double* b, double* x, int* Iarray, double* Rarray,
                                int reps, int* best, double* ms);

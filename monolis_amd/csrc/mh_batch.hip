@@ -594,9 +594,12 @@ __global__ void k_batch_fill(int nsys_rows_total, const int* __restrict__ sell_s
 // 10^3..40^3 rows: 17.6 ms against 51.1 for the best of the others (the
 // vectors' 108 of 190 bytes per row and iteration stay on chip).  It is the
 // default of every batch it fits; one with a system it does not fit runs
-// kCfgFallback instead (also when configuration 15 is asked for).
+// kCfgFallback instead (also when configuration 15 is asked for).  A solve of
+// which a team gave up waiting is redone with kCfgNoTeams, where nothing waits
+// for another workgroup, and so are the following ones (Batch::res_off).
 constexpr int kCfgResident = 15;
 constexpr int kCfgFallback = 11;
+constexpr int kCfgNoTeams = 0;
 
 // Team schedule of a configuration (NT threads per workgroup, `resident`
 // workgroups at once, split factor ts): the estimated work of a system is
@@ -706,7 +709,8 @@ static int ensure_sched(Batch& B, int cfg, BatchSched** out, hipStream_t s) {
 
 // The configuration that a launch of cfg runs.
 static int effective_config(const Batch& B, int cfg) {
-  return cfg == kCfgResident && !B.res.fits ? kCfgFallback : cfg;
+  if (cfg != kCfgResident) return cfg;
+  return !B.res.fits ? kCfgFallback : B.res_off ? kCfgNoTeams : cfg;
 }
 
 int batch_schedule_info(Batch& B, int cfg, int* split, int* nslot, int* nteam, hipStream_t s) {
@@ -936,6 +940,26 @@ int batch_solve(Batch& B, const BatchParams& P, const double* b, double* x, int 
     B.g_wait = B.wait_s;
   }
   MH_HIP(hipGraphLaunch(B.graph_exec, s));
+  return 0;
+}
+
+bool batch_leave_chip(Batch& B) {
+  if (effective_config(B, B.cfg) != kCfgResident) return false;
+  B.res_off = true;
+  return true;
+}
+
+int batch_solve_safe(Batch& B, const BatchParams& P, const double* b, double* x, int* aborted, hipStream_t s) {
+  double* x0 = B.work.p;  // the on-chip solver leaves this part of the work vectors alone
+  const bool keep = effective_config(B, B.cfg) == kCfgResident && !P.init_x && B.res.nteam > 0;
+  if (keep) MH_HIP(hipMemcpyAsync(x0, x, sizeof(double) * (size_t)B.n, hipMemcpyDeviceToDevice, s));
+  MH_TRY(batch_solve(B, P, b, x, B.cfg, 1, s));
+  MH_TRY(batch_aborted(B, B.cfg, aborted, s));
+  if (!*aborted || !batch_leave_chip(B)) return 0;
+  *aborted = 0;
+  if (keep) MH_HIP(hipMemcpyAsync(x, x0, sizeof(double) * (size_t)B.n, hipMemcpyDeviceToDevice, s));
+  MH_TRY(batch_solve(B, P, b, x, B.cfg, 0, s));
+  MH_HIP(hipStreamSynchronize(s));
   return 0;
 }
 

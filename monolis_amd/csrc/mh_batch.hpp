@@ -43,6 +43,7 @@ struct Batch {
   ResPlan res;  // on-chip solver's members (res.fits: usable)
   int cfg = 0;  // launch configuration: the on-chip solver where it fits, 0 otherwise, or the tuned one
   double wait_s = 5.0;  // longest team wait before a launch gives up
+  bool res_off = false; // an on-chip team gave up: no teams until the limit or the configuration is set again
   // captured launch (replayed while arguments are unchanged)
   hipGraphExec_t graph_exec = nullptr;
   const double* g_b = nullptr;
@@ -62,6 +63,11 @@ int batch_create(Batch** out, int nsys, const int* sys_row_host, int n, int nz, 
                  const double* A, hipStream_t s);
 // Enqueues one batched solve (graph replay when use_graph); results in B.iters/resid/status.
 int batch_solve(Batch& B, const BatchParams& P, const double* b, double* x, int cfg, int use_graph, hipStream_t s);
+// The same with the batch's own configuration (graph replay), completed on return.
+// An on-chip solve of which a team gave up waiting is redone from the same start
+// vector without teams; *aborted = 1: a team of another configuration gave up.
+bool batch_leave_chip(Batch& B);  // Ends on-chip solves of B (res_off); false: its configuration does not run there.
+int batch_solve_safe(Batch& B, const BatchParams& P, const double* b, double* x, int* aborted, hipStream_t s);
 // After launches of configuration cfg have completed: 1 when a team wait gave up
 // in any of them since the last call (the affected systems carry status 3), else 0.
 int batch_aborted(Batch& B, int cfg, int* aborted, hipStream_t s);

@@ -873,6 +873,7 @@ int monolis_hip_batch_set_config(monolis_hip_batch* H, int cfg) {
     mh::set_error("batch config %d out of range", cfg);
     return ST_ARGS;
   }
+  H->B->res_off = false;
   H->B->cfg = cfg;
   return 0;
 }
@@ -894,6 +895,7 @@ int monolis_hip_batch_set_wait_limit(monolis_hip_batch* H, double seconds) {
     return ST_ARGS;
   }
   H->B->wait_s = seconds;
+  H->B->res_off = false;
   return 0;
 }
 
@@ -905,14 +907,13 @@ int monolis_hip_batch_solve(monolis_hip_batch* H, const double* b, double* x, in
   if (rc0) return rc0;
   const double t0 = now();
   mh::Batch& B = *H->B;
-  MH_TRY(mh::batch_solve(B, batch_params(Iarray, Rarray), b, x, B.cfg, 1, c->stream));
+  int aborted = 0;
+  MH_TRY(mh::batch_solve_safe(B, batch_params(Iarray, Rarray), b, x, &aborted, c->stream));
   MH_HIP(hipStreamSynchronize(c->stream));
   if (iters) MH_HIP(hipMemcpy(iters, B.iters.p, sizeof(int) * B.nsys, hipMemcpyDeviceToHost));
   if (resid) MH_HIP(hipMemcpy(resid, B.resid.p, sizeof(double) * B.nsys, hipMemcpyDeviceToHost));
   if (status) MH_HIP(hipMemcpy(status, B.status.p, sizeof(int) * B.nsys, hipMemcpyDeviceToHost));
   Rarray[R_TIME_SOL] = now() - t0;
-  int aborted = 0;
-  MH_TRY(mh::batch_aborted(B, B.cfg, &aborted, c->stream));
   if (aborted) {
     mh::set_error("batched solve: a team of workgroups gave up waiting for a member (systems with status 3)");
     return ST_HIP;
@@ -928,21 +929,27 @@ int monolis_hip_batch_time(monolis_hip_batch* H, const double* b, double* x, int
   if (rc0) return rc0;
   mh::Batch& B = *H->B;
   const mh::BatchParams P = batch_params(Iarray, Rarray);
-  MH_TRY(mh::batch_solve(B, P, b, x, B.cfg, 1, c->stream));  // capture + warm-up
+  int aborted = 0;
+  MH_TRY(mh::batch_solve_safe(B, P, b, x, &aborted, c->stream));  // capture + warm-up
   hipEvent_t e0, e1;
   MH_HIP(hipEventCreate(&e0));
   MH_HIP(hipEventCreate(&e1));
-  MH_HIP(hipEventRecord(e0, c->stream));
-  for (int i = 0; i < reps; ++i) MH_TRY(mh::batch_solve(B, P, b, x, B.cfg, 1, c->stream));
-  MH_HIP(hipEventRecord(e1, c->stream));
-  MH_HIP(hipEventSynchronize(e1));
+  for (int late = 1; late;) {
+    MH_HIP(hipEventRecord(e0, c->stream));
+    for (int i = 0; i < reps; ++i) MH_TRY(mh::batch_solve(B, P, b, x, B.cfg, 1, c->stream));
+    MH_HIP(hipEventRecord(e1, c->stream));
+    MH_HIP(hipEventSynchronize(e1));
+    MH_TRY(mh::batch_aborted(B, B.cfg, &late, c->stream));
+    if (late && !mh::batch_leave_chip(B)) {  // on chip: timed again without teams
+      aborted = 1;
+      break;
+    }
+  }
   float t = 0.f;
   MH_HIP(hipEventElapsedTime(&t, e0, e1));
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   *ms = reps > 0 ? (double)t / reps : 0.0;
-  int aborted = 0;
-  MH_TRY(mh::batch_aborted(B, B.cfg, &aborted, c->stream));
   if (aborted) {
     mh::set_error("batched solve: a team of workgroups gave up waiting for a member");
     return ST_HIP;
@@ -960,6 +967,7 @@ int monolis_hip_batch_autotune(monolis_hip_batch* H, const double* b, double* x,
   const mh::BatchParams P = batch_params(Iarray, Rarray);
   double best_ms = 1e300;
   int best_cfg = 0;
+  B.res_off = false;
   for (int cfg = 0; cfg < mh::batch_num_configs(); ++cfg) {
     MH_TRY(mh::batch_solve(B, P, b, x, cfg, 0, c->stream));  // warm-up
     hipEvent_t e0, e1;

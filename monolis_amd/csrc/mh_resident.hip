@@ -102,15 +102,17 @@ __global__ void __launch_bounds__(kResNT) k_res_build(ResMember* mem, const int*
 }
 
 // Per-launch reset (a kernel, so that a captured graph holds no memset nodes).
-__global__ void k_res_reset(int nsys, int* iters, double* resid, int* status, int* ctl, unsigned long long* part,
-                            int npart) {
+// `abort`: no member of a team may wait at all.
+__global__ void k_res_reset(int nsys, int* iters, double* resid, int* status, int* ctl, int abort, int* sticky,
+                            unsigned long long* part, int npart) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < nsys) {
     iters[i] = -1;
     resid[i] = 0.0;
     status[i] = -1;
   }
-  if (i < 2) ctl[i] = 0;
+  if (i < 2) ctl[i] = i == 1 ? abort : 0;
+  if (i == 0 && abort) *sticky = 1;
   if (i < npart) part[i] = 0;  // no tag of an earlier launch
 }
 
@@ -266,7 +268,8 @@ int res_launch(const ResPlan& plan, const int* d_slice_ptr, const double* val, c
                int nsys, double wait_s, hipStream_t s) {
   const int npart = plan.nteam * 8 * kResTeamMax;
   k_res_reset<<<(std::max(nsys, npart + 2) + kBlock - 1) / kBlock, kBlock, 0, s>>>(
-      nsys, a.out.iters, a.out.resid, a.out.status, plan.ctl.p, plan.part.p, npart);
+      nsys, a.out.iters, a.out.resid, a.out.status, plan.ctl.p, plan.nteam > 0 && wait_s == 0.0, plan.sticky.p,
+      plan.part.p, npart);
   MH_HIP(hipGetLastError());
   const ResView V{plan.nmem, (const ResMember*)plan.mem.p, d_slice_ptr, plan.g_ptr.p, val, (const uint4*)plan.lcol.p,
                   plan.expf.p, dinv, plan.halo.p, plan.ctl.p, plan.part.p, (long long)(plan.ticks_per_s * wait_s),

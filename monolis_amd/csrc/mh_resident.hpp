@@ -91,7 +91,7 @@ struct ResArgs {
 struct ResShared {
   double red[2][2 * kResNW];
   double tot[2];
-  int ok, next;
+  int ok, next, aborted;
 };
 
 __device__ __forceinline__ void st_agent(double* p, double v) {
@@ -485,19 +485,26 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
 // Persistent: workgroups take members in order from one counter.  A team's
 // members are consecutive, so at most one team is incomplete at any time and a
 // member waiting for a teammate that has not started waits only for running
-// workgroups to finish their own complete teams.
+// workgroups to finish their own complete teams.  Members of teams that start
+// after a wait gave up report it at once.
 template <int RP, bool MR>
 __global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP <= kResRowsSmall && !MR ? 4 : 2)))
     k_res_cg(ResView V, ResArgs a) {
   extern __shared__ double res_lds[];
   __shared__ ResShared sh;
   for (;;) {
-    if (threadIdx.x == 0) sh.next = __hip_atomic_fetch_add(V.ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (threadIdx.x == 0) {
+      sh.next = __hip_atomic_fetch_add(V.ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sh.aborted = __hip_atomic_load(V.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     __syncthreads();
     const int k = __builtin_amdgcn_readfirstlane(sh.next);
     if (k >= V.nmem) break;
     const ResMember m = V.mem[k];
-    if constexpr (MR) {
+    if (m.T > 1 && __builtin_amdgcn_readfirstlane(sh.aborted) != 0) {
+      if (threadIdx.x == 0)
+        __hip_atomic_fetch_max(a.out.status + m.sys, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else if constexpr (MR) {
       res_cg<RP, true, true>(V, m, a, res_lds, sh);
     } else {
       if (m.w8) res_cg<RP, true, false>(V, m, a, res_lds, sh);
@@ -532,7 +539,8 @@ struct ResPlan {
 int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
                    const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int team_limit,
                    hipStream_t s);
-// Zeroes the counters and enqueues the solver (both capturable).
+// Zeroes the counters and enqueues the solver (both capturable).  A wait of a
+// team's member for another lasts at most wait_s seconds; 0: teams give up at once.
 int res_launch(const ResPlan& plan, const int* d_slice_ptr, const double* val, const double* dinv, const ResArgs& a,
                int nsys, double wait_s, hipStream_t s);
 // 1 when a team wait gave up in any launch since the last call (synchronises).

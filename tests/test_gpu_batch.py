@@ -343,16 +343,50 @@ def test_on_chip_batch_that_does_not_fit_runs_another_configuration():
     _check_against_oracle(mat, sys_row, b, dx.numpy(), iters, resid, status)
 
 
-def test_on_chip_wait_limit_gives_up_cleanly():
+@pytest.mark.parametrize("init_x", [True, False])
+def test_on_chip_wait_limit_gives_up_cleanly(init_x):
+    """With limit 0 every team gives up at its start: the batch is then solved without teams, from the same
+    start vector (12 iterations of the oracle from there), and stays so until the limit is set again."""
     mat, sys_row = W.poisson_batch(edges=[30, 24, 9])
+    b, x0 = W.uniform_vector(mat.n, seed=4), W.uniform_vector(mat.n, seed=5)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
+    B = api.DeviceBatch(mat, sys_row)
+    assert B.schedule(ON_CHIP)["teams"] >= 1
+    B.set_wait_limit(0.0)
+    prm = _prm(max_iter=12)
+    prm.Iarray[api.MONOLIS_PRM_I_IS_INIT_X] = int(init_x)
+    for _ in range(2):                               # gives up; already without teams
+        dx.upload(x0)
+        iters, resid, status = B.solve(db, dx, prm)
+        assert B.schedule(ON_CHIP) == {"split": 0, "slots": 3, "teams": 0}
+        x = dx.numpy()
+        for k in range(3):
+            s = slice(sys_row[k], sys_row[k + 1])
+            I, R = oracle.default_arrays(max_iter=12)
+            I[10] = int(init_x)
+            xo, st, I, R = oracle.solve(_system(mat, sys_row, k), b[s], x0=x0[s], Iarray=I, Rarray=R)
+            assert status[k] == (1 if st else 0) and iters[k] == int(I[4])
+            assert np.linalg.norm(x[s] - xo) <= 1e-9 * np.linalg.norm(xo)
+    assert B.time(db, dx, prm, reps=2) > 0
+    B.set_wait_limit(0.0)                            # set again: on chip, and gives up while timed
+    assert B.schedule(ON_CHIP)["split"] == 1
+    assert B.time(db, dx, prm, reps=2) > 0
+    assert B.schedule(ON_CHIP)["split"] == 0
+    B.set_wait_limit(5.0)
+    assert B.schedule(ON_CHIP)["split"] == 1
+    iters, resid, status = B.solve(db, dx, _prm())
+    assert B.schedule(ON_CHIP)["split"] == 1
+    _check_against_oracle(mat, sys_row, b, dx.numpy(), iters, resid, status)
+
+
+def test_on_chip_give_up_in_autotuning_leaves_the_other_configurations():
+    mat, sys_row = W.poisson_batch(edges=[24, 9])
     b = W.uniform_vector(mat.n, seed=4)
     db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
     B = api.DeviceBatch(mat, sys_row)
     B.set_wait_limit(0.0)
-    try:
-        B.solve(db, dx, _prm())
-    except RuntimeError as e:
-        assert "gave up" in str(e)
+    t = B.autotune(db, dx, _prm(), reps=1)
+    assert t["best"] != ON_CHIP and t["ms"][ON_CHIP] >= 1e29
     B.set_wait_limit(5.0)
     iters, resid, status = B.solve(db, dx, _prm())
     _check_against_oracle(mat, sys_row, b, dx.numpy(), iters, resid, status)
