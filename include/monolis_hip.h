@@ -202,9 +202,18 @@ int monolis_hip_matrix_autotune(monolis_hip_matrix* M, int fp32, int reps, int* 
  * The timed solves take the launch-per-step solver, whose SpMV the variant is. */
 int monolis_hip_matrix_autotune_solver(monolis_hip_matrix* M, int fp32, int method, int precond, int iters,
                                        int reps, int* best, double* ms);
-/* Solves of the handle so far that ran in one launch with the vectors on chip
- * (FP64 CG on scalar systems that fit; the SpMV variant plays no part there). */
-int monolis_hip_matrix_on_chip_solves(const monolis_hip_matrix* M, int* solves);
+/* FP64 CG on a scalar system that fits runs in one launch with the vectors on
+ * chip, by workgroups that wait for one another (the SpMV variant plays no part
+ * there).  on = 0 keeps the handle's solves to the launch-per-step solver.
+ * wait_s (default 0.5, at most 600) is the longest time in seconds that one
+ * workgroup waits for another, which other work on the GPU may keep from
+ * starting: the solve is then redone launch by launch from the same start vector,
+ * and the handle's later solves are not tried on chip until this call is made
+ * again.  With wait_s = 0 every solve by more than one workgroup gives up. */
+int monolis_hip_matrix_set_on_chip(monolis_hip_matrix* M, int on, double wait_s);
+/* Solves of the handle and its transpose so far that ran on chip, and those of
+ * which a wait gave up. */
+int monolis_hip_matrix_on_chip_solves(const monolis_hip_matrix* M, int* solves, int* gave_up);
 /* Forces a variant for one precision (fp32 = 0 or 1); an untuned handle uses
  * variant 4 (one wavefront per slice, 3 slots per step). */
 int monolis_hip_matrix_set_variant(monolis_hip_matrix* M, int fp32, int variant);

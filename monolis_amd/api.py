@@ -12,7 +12,7 @@ device-resident extension.
 from __future__ import annotations
 
 import ctypes
-from typing import Optional
+from typing import Optional, Tuple
 
 import numpy as np
 
@@ -432,12 +432,18 @@ class DeviceMatrix:
                    "autotune_solver")
         return {"best": best.value, "ms_per_iter": list(ms)}
 
-    def on_chip_solves(self) -> int:
-        """Solves of this handle so far that ran in one launch with the vectors on chip."""
-        n = ctypes.c_int()
-        _lib.check(_lib.load().monolis_hip_matrix_on_chip_solves(ctypes.c_void_p(self.h), ctypes.byref(n)),
-                   "on_chip_solves")
-        return n.value
+    def set_on_chip(self, on: bool = True, wait_s: float = 0.5) -> None:
+        """Whether FP64 CG on a scalar system may run in one launch with the vectors on chip, and how long one
+        of its workgroups waits for another before the solve is redone launch by launch."""
+        _lib.check(_lib.load().monolis_hip_matrix_set_on_chip(ctypes.c_void_p(self.h), int(on), float(wait_s)),
+                   "set_on_chip")
+
+    def on_chip_solves(self) -> Tuple[int, int]:
+        """Solves so far that ran on chip, and those of which a wait gave up."""
+        n, g = ctypes.c_int(), ctypes.c_int()
+        _lib.check(_lib.load().monolis_hip_matrix_on_chip_solves(ctypes.c_void_p(self.h), ctypes.byref(n),
+                                                                 ctypes.byref(g)), "on_chip_solves")
+        return n.value, g.value
 
     def set_variant(self, variant: int, fp32: bool = False) -> None:
         _lib.check(_lib.load().monolis_hip_matrix_set_variant(ctypes.c_void_p(self.h), int(fp32), int(variant)),

@@ -173,6 +173,8 @@ int matrix_transpose(Matrix* M, hipStream_t s) {
     Matrix* T = nullptr;
     MH_TRY(matrix_create(&T, n, n, nz, b, rowptrT.p, itemT.p, AT.p, s));
     MH_HIP(hipStreamSynchronize(s));  // temporaries are released on return
+    T->on_chip = M->on_chip;
+    T->on_chip_wait = M->on_chip_wait;
     M->transpose = T;
     M->transpose_stale = false;
     return 0;

@@ -802,12 +802,30 @@ int monolis_hip_matrix_autotune_solver(monolis_hip_matrix* H, int fp32, int meth
   return rc ? (rc == -3 ? ST_PRECOND : rc == -4 ? ST_METHOD : rc == -2 ? ST_ARGS : ST_HIP) : 0;
 }
 
-int monolis_hip_matrix_on_chip_solves(const monolis_hip_matrix* H, int* solves) {
-  if (!H || !H->M || !solves) {
+int monolis_hip_matrix_set_on_chip(monolis_hip_matrix* H, int on, double wait_s) {
+  if (!H || !H->M || !(wait_s >= 0.0) || wait_s > 600.0) {
+    mh::set_error("set_on_chip: needs a matrix handle and a wait limit in [0, 600] s");
+    return ST_ARGS;
+  }
+  for (Matrix* M : {H->M, H->M->transpose})
+    if (M) {
+      M->on_chip = on != 0;
+      M->on_chip_wait = wait_s;
+    }
+  return 0;
+}
+
+int monolis_hip_matrix_on_chip_solves(const monolis_hip_matrix* H, int* solves, int* gave_up) {
+  if (!H || !H->M || !solves || !gave_up) {
     mh::set_error("on_chip_solves: null argument");
     return ST_ARGS;
   }
-  *solves = H->M->on_chip_solves;
+  *solves = *gave_up = 0;
+  for (const Matrix* M : {(const Matrix*)H->M, (const Matrix*)H->M->transpose})
+    if (M) {
+      *solves += M->on_chip_solves;
+      *gave_up += M->on_chip_gave_up;
+    }
   return 0;
 }
 

@@ -156,7 +156,9 @@ struct Matrix {
   bool transpose_stale = false;   // values of A changed since the transpose was filled
   VBlock* vb = nullptr;           // non-null for variable block sizes
   ResPlan* res = nullptr;         // built by the first solve that may run on chip
-  int on_chip_solves = 0;         // solves that ran on chip
+  bool on_chip = true;            // solves may run on chip (ends with a wait that gives up)
+  double on_chip_wait = 0.5;      // longest wait of one workgroup for another, seconds
+  int on_chip_solves = 0, on_chip_gave_up = 0;  // solves that ran on chip; solves of which a wait gave up
   // complex matrices (monolis's *_C path): values in valz instead of val64,
   // complex block-Jacobi factors in Dz (same structure-of-arrays layout as D64)
   bool is_complex = false;

@@ -1286,12 +1286,16 @@ size_t cg_bytes(const Matrix& M, int nvec, int max_iter) {
 
 // The on-chip CG on a scalar system (mh_resident.hpp): one launch instead of
 // three per iteration.  *ran stays false when the system does not fit, or when
-// a team's wait gave up (x is then as it was); the launch-per-step solver
-// follows.  Solves with a time split take that one too: it times its steps.
+// a team's wait gave up (x is then as it was, and the matrix's later solves no
+// longer try); the launch-per-step solver follows.  Solves with a time split take
+// that one too: it times its steps.
+// A team needs all of its workgroups (at most 128) on the GPU at once, which other
+// work on it can prevent: the wait limit is what that may cost a matrix, once
+// (0.5 s by default, against at most about 50 us between two exchanges).
 int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, double* x, Workspace& W,
                SolveResult* out, bool* ran, hipStream_t s) {
   *ran = false;
-  if (M.n < 1 || M.n != M.np || P.max_iter < 1 || P.steps || active_ktimer()) return 0;
+  if (M.n < 1 || M.n != M.np || P.max_iter < 1 || P.steps || !M.on_chip || active_ktimer()) return 0;
   if ((long long)M.nslices > (long long)kResTeamMax * kResRowsLarge * kResNW) return 0;
   if (!M.res) {
     M.res = new ResPlan();
@@ -1320,11 +1324,13 @@ int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, doub
   if (!P.init_x) MH_HIP(hipMemcpyAsync(x0, x, m * sizeof(double), hipMemcpyDeviceToDevice, s));
   const ResArgs a{b, x, z, p, xe, {&d->iter, &d->resid, &d->status}, P.keep_hist ? hist : nullptr, P.max_iter, P.tol,
                   P.init_x, prec ? 1 : 0};
-  MH_TRY(res_launch(*M.res, M.slice_ptr.p, M.val64.p, prec ? M.D64.p : nullptr, a, 1, 5.0, s));
+  MH_TRY(res_launch(*M.res, M.slice_ptr.p, M.val64.p, prec ? M.D64.p : nullptr, a, 1, M.on_chip_wait, s));
   MH_HIP(hipMemcpyAsync(&h, d, sizeof(Result), hipMemcpyDeviceToHost, s));
   MH_HIP(hipStreamSynchronize(s));
   if (h.status < 0 || h.status > 2) {
     int gave_up = 0;
+    ++M.on_chip_gave_up;
+    M.on_chip = false;
     MH_TRY(res_aborted(*M.res, &gave_up, s));
     if (!P.init_x) MH_HIP(hipMemcpyAsync(x, x0, m * sizeof(double), hipMemcpyDeviceToDevice, s));
     return 0;

@@ -135,11 +135,11 @@ def test_solver_tuning_times_the_launches_that_the_variant_is_of():
     dm = api.DeviceMatrix(mat)
     for precond in (1, 0):
         t = dm.autotune_solver(fp32=False, precond=precond, iters=6, reps=1)
-        assert dm.on_chip_solves() == 0
+        assert dm.on_chip_solves() == (0, 0)
         assert all(v > 0 for v in t["ms_per_iter"]) and t["ms_per_iter"][t["best"]] == min(t["ms_per_iter"])
     db, dx = api.DeviceBuffer.from_numpy(W.uniform_vector(3000, seed=1)), api.DeviceBuffer(3000)
     dm.solve(db, dx, _prm())
-    assert dm.on_chip_solves() == 1
+    assert dm.on_chip_solves() == (1, 0)
 
 
 def test_on_chip_handles_of_one_kernel_and_different_lds():
@@ -159,7 +159,7 @@ def test_on_chip_handles_of_one_kernel_and_different_lds():
         b[0].solve(b[1], b[2], _prm())
         a[2].upload(np.zeros(big.n))
         a[0].solve(a[1], a[2], _prm())
-        assert a[0].on_chip_solves() == 2 and b[0].on_chip_solves() == 1
+        assert a[0].on_chip_solves() == (2, 0) and b[0].on_chip_solves() == (1, 0)
         assert np.array_equal(x, a[2].numpy())
     out = []
     for edges in ([40, 40, 38], [8, 9]):
@@ -173,3 +173,51 @@ def test_on_chip_handles_of_one_kernel_and_different_lds():
     dx.upload(np.zeros(len(x)))
     B.solve(db, dx, _prm())
     assert np.array_equal(x, dx.numpy())
+
+
+@pytest.mark.parametrize("init_x", [True, False])
+def test_on_chip_wait_that_gives_up_is_redone_by_steps(init_x):
+    """With wait limit 0 a team gives up at its start: the solve is redone launch by launch from the same start
+    vector, the next ones take that solver at once, and setting the limit again brings the team back."""
+    mat = W.poisson7(32)
+    b, x0 = W.uniform_vector(mat.n, seed=3), W.uniform_vector(mat.n, seed=4)
+    I, R = oracle.default_arrays(max_iter=12)
+    I[10] = int(init_x)
+    xo, st, I, R = oracle.solve(mat, b, x0=x0, Iarray=I, Rarray=R)
+    dm = api.DeviceMatrix(mat)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
+
+    def check(solves, gave_up):
+        dx.upload(x0)
+        prm = _prm(max_iter=12, init_x=init_x)
+        h = dm.solve(db, dx, prm, hist_len=20)
+        assert dm.on_chip_solves() == (solves, gave_up)
+        assert int(prm.Iarray[api.MONOLIS_PRM_I_IERR]) == st and int(prm.Iarray[api.MONOLIS_PRM_I_CUR_ITER]) == 12
+        assert h[12] == prm.Rarray[api.MONOLIS_PRM_R_CUR_RESID] and np.linalg.norm(dx.numpy() - xo) <= 1e-9 * np.linalg.norm(xo)
+
+    check(1, 0)
+    dm.set_on_chip(True, 0.0)
+    check(1, 1)
+    check(1, 1)
+    dm.set_on_chip(True, 5.0)
+    check(2, 1)
+    dm.set_on_chip(False)
+    check(2, 1)
+    with pytest.raises(RuntimeError):
+        dm.set_on_chip(True, -1.0)
+
+
+def test_on_chip_settings_reach_the_transpose():
+    mat = _matrix(3000, 500, False, 12)      # symmetric: the solution of A^T x = b is that of A x = b
+    dm = api.DeviceMatrix(mat)
+    db, dx = api.DeviceBuffer.from_numpy(W.uniform_vector(3000, seed=1)), api.DeviceBuffer(3000)
+    dm.set_on_chip(False)
+    dm.solve_transpose(db, dx, _prm())
+    assert dm.on_chip_solves() == (0, 0)
+    xs = dx.numpy()
+    dm.set_on_chip(True, 0.0)
+    dm.solve_transpose(db, dx, _prm())
+    assert dm.on_chip_solves() == (0, 1) and np.array_equal(xs, dx.numpy())
+    dm.set_on_chip(True)
+    dm.solve_transpose(db, dx, _prm())
+    assert dm.on_chip_solves() == (1, 1) and np.linalg.norm(dx.numpy() - xs) <= 1e-6 * np.linalg.norm(xs)
