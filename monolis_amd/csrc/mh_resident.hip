@@ -7,8 +7,6 @@
 
 namespace mh {
 
-int cu_count();
-
 namespace {
 
 // One workgroup per member: marks the columns outside the member's rows in a
@@ -135,7 +133,7 @@ int occupancy(size_t lds, int* per_cu) {
 }  // namespace
 
 int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
-                   const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int team_limit,
+                   const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int cus,
                    hipStream_t s) {
   plan.fits = false;
   double W = 0.0;
@@ -153,19 +151,8 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
   std::vector<Task> tasks;
   for (size_t k = 0; k < sys.size(); ++k) {
     const ResSystem& q = sys[k];
-    if (q.rows == 0) return 0;
-    const int need = (q.nsl + kResRowsLarge * kResNW - 1) / (kResRowsLarge * kResNW);
-    // More members than capacity asks for, while the system's share of the
-    // workgroups allows: down to one row per thread (7-point systems, us per
-    // iteration with 64 / 128 members: 48^3 10.3 / 8.1, 64^3 19.7 / 11.2, 78^3
-    // 34.8 / 19.8; 32^3 is flat from 32 to 128 at 7.0-7.3).  Up to four rows per
-    // thread one workgroup alone is faster (10^3: 4.0 against 5.7 with four
-    // members, 12^3: 4.5 against 6.0): a team's two exchanges cost about 1 us each.
-    const int fair = (int)((double)team_limit * q.work / std::max(W, 1e-300));
-    int T = std::max(need, std::min(std::min(kResTeamMax, fair), q.nsl / kResNW));
-    if (need == 1 && q.nsl <= kResRowsMini * kResNW) T = 1;
-    T = std::max(T, 1);
-    if (T > kResTeamMax) return 0;
+    const int T = res_members(q.nsl, (int)((double)cus * q.work / std::max(W, 1e-300)), cus);
+    if (T == 0) return 0;
     tasks.push_back(Task{(int)k, T, ((double)q.rows / T + 1500.0) * std::cbrt((double)q.rows)});
   }
   std::stable_sort(tasks.begin(), tasks.end(), [](const Task& a, const Task& b) { return a.d > b.d; });
@@ -255,7 +242,7 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
   else if (plan.rp == kResRowsSmall) MH_TRY((occupancy<kResRowsSmall, false>(plan.lds_bytes, &per_cu)));
   else MH_TRY((occupancy<kResRowsLarge, false>(plan.lds_bytes, &per_cu)));
   if (per_cu < 1) return 0;
-  plan.grid = std::min(plan.nmem, per_cu * cu_count());
+  plan.grid = std::min(plan.nmem, per_cu * cus);
   int dev = 0, khz = 0;
   MH_HIP(hipGetDevice(&dev));
   if (hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, dev) != hipSuccess || khz <= 0) khz = 100000;

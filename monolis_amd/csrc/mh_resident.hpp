@@ -28,18 +28,13 @@
 
 #include "mh_internal.hpp"
 #include "mh_kernels.hpp"
+#include "mh_resident_plan.hpp"
 
 namespace mh {
 
-constexpr int kResNT = 512;                 // threads per member: two wavefronts per SIMD, 256 VGPRs each
-constexpr int kResNW = kResNT / kWave;
-constexpr int kResTeamMax = 128;            // workgroups per team at most (one wavefront polls 4 words of each)
 constexpr int kResLds = 20320;              // doubles of LDS for p (158.75 KB of the CU's 160)
 constexpr int kResSpinMax = 1 << 24;        // polls of one team wait at most (a bound that needs no clock)
 constexpr int kResIterRR = 200;             // residual replacement (CG.f90:91-95)
-constexpr int kResRowsLarge = 26;           // RP: 13,312 rows per member (150 VGPRs of vectors)
-constexpr int kResRowsMini = 4;             // RP: 2,048 rows
-constexpr int kResRowsSmall = 8;            // RP: 4,096 rows (with the matrix in registers: 208 VGPRs of data)
 
 struct ResMember {
   int sys, rank, T, team;
@@ -534,10 +529,11 @@ struct ResPlan {
 
 // slice_ptr: host slot offsets of every slice; d_slice_ptr / d_col: the device
 // arrays (global 0-based columns); rowlen (per SELL row) or rowptr (per row)
-// gives the row lengths.  Plan.fits is false when a system needs more than
-// kResTeamMax members or a member's rows and halo exceed LDS.
+// gives the row lengths.  Plan.fits is false when a system needs more members than
+// a team may have or a member's rows and halo exceed LDS.  cus: the GPU's CUs, the
+// workgroups that the systems share.
 int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
-                   const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int team_limit,
+                   const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int cus,
                    hipStream_t s);
 // Zeroes the counters and enqueues the solver (both capturable).  A wait of a
 // team's member for another lasts at most wait_s seconds; 0: teams give up at once.
