@@ -113,6 +113,11 @@ void* monolis_hip_stream(void);
 int monolis_hip_synchronize(void);
 int monolis_hip_malloc(void** ptr, size_t bytes);
 int monolis_hip_free(void* ptr);
+/* The library keeps device blocks that it has released, at most 4 GiB, for its
+ * next allocations.  This gives them back to the GPU (another allocator in the
+ * process may need them; monolis_hip_malloc does it by itself when it must);
+ * bytes, if not NULL, receives how much that was. */
+int monolis_hip_trim(unsigned long long* bytes);
 /* Copy in any direction (host/device detected from the pointers), synchronous. */
 int monolis_hip_memcpy(void* dst, const void* src, size_t bytes);
 int monolis_hip_memset(void* dst, int value, size_t bytes);

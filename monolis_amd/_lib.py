@@ -62,6 +62,7 @@ SIGNATURES = [
     ("monolis_hip_synchronize", c_int, []),
     ("monolis_hip_malloc", c_int, [ctypes.POINTER(c_void_p), c_size_t]),
     ("monolis_hip_free", c_int, [c_void_p]),
+    ("monolis_hip_trim", c_int, [ctypes.POINTER(ctypes.c_ulonglong)]),
     ("monolis_hip_memcpy", c_int, [c_void_p, c_void_p, c_size_t]),
     ("monolis_hip_memset", c_int, [c_void_p, c_int, c_size_t]),
     ("monolis_hip_matrix_create", c_int, [ctypes.POINTER(c_void_p), c_int, c_int, c_int, c_int,

@@ -196,6 +196,13 @@ def monolis_inner_product_C(monolis: Monolis, n_dof: int, x: np.ndarray, y: np.n
 # ---------------------------------------------------------------------------
 # device-resident interface
 # ---------------------------------------------------------------------------
+def trim() -> int:
+    """Gives the device blocks that the library keeps for its next allocations back to the GPU; returns their bytes."""
+    n = ctypes.c_ulonglong()
+    _lib.check(_lib.load().monolis_hip_trim(ctypes.byref(n)), "monolis_hip_trim")
+    return n.value
+
+
 class DeviceBuffer:
     """A device allocation owned by Python (freed with the object)."""
 

@@ -414,7 +414,12 @@ int monolis_hip_synchronize(void) {
 int monolis_hip_malloc(void** ptr, size_t bytes) {
   Context* c = nullptr;
   MH_TRY(mh::context(&c));
-  MH_HIP(hipMalloc(ptr, bytes ? bytes : 1));
+  return mh::dev_alloc_outside(ptr, bytes ? bytes : 1);
+}
+
+int monolis_hip_trim(unsigned long long* bytes) {
+  const size_t n = mh::dev_trim();
+  if (bytes) *bytes = n;
   return 0;
 }
 

@@ -50,6 +50,10 @@ Context* context_if_ready();
 // handed back to dev_free, which keeps the block for a later allocation.
 int dev_alloc(void** p, size_t bytes, size_t* cap);
 void dev_free(void* p, size_t cap);
+// hipMalloc that may need the blocks the library keeps (user buffers).
+int dev_alloc_outside(void** p, size_t bytes);
+// Gives every kept block back; returns their bytes.
+size_t dev_trim();
 
 template <typename T>
 struct DevArray {

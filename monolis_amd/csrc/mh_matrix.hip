@@ -3,13 +3,13 @@
 #include <cstdio>
 #include <cstring>
 #include <algorithm>
-#include <map>
 #include <mutex>
 #include <thread>
 #include <vector>
 
 #include "mh_internal.hpp"
 #include "mh_launch.hpp"
+#include "mh_pool.hpp"
 #include "mh_resident.hpp"
 
 namespace mh {
@@ -61,96 +61,36 @@ Context* context_if_ready() {
   return g_ctx.ok ? &g_ctx : nullptr;
 }
 
-// Released device blocks kept for the next allocation.  hipMalloc + hipFree take
-// 0.1-0.3 ms a pair here and hipFree waits for the device: the 35 temporaries of
-// one 64^3-hexahedra assembly took 5.9 of its 7.8 ms.  Every block is used on
-// the library's one stream (the upload streams wait for it first), so a block
-// handed on while earlier work is still enqueued is safe by stream order, from
-// any thread.  At most kPoolBytes stay cached -- about 1.5 % of the GPU's memory;
-// past that the largest go back at once, and all of them when an allocation
-// fails.  Blocks of other devices than the first one used are never kept.
 namespace {
+// About 1.5 % of the GPU's memory.
 constexpr size_t kPoolBytes = (size_t)4 << 30;
-struct DevPool {
-  std::mutex mu;
-  std::multimap<size_t, void*> blocks;  // by size
-  size_t cached = 0;
-  int device = -1;
+thread_local hipError_t g_alloc_err = hipSuccess;  // of this thread's last allocation
+struct HipMem {
+  bool alloc(void** p, size_t bytes) {
+    g_alloc_err = hipMalloc(p, bytes);
+    if (g_alloc_err != hipSuccess) (void)hipGetLastError();
+    return g_alloc_err == hipSuccess;
+  }
+  void free(void* p) { (void)hipFree(p); }
 };
-DevPool& pool() {
-  static DevPool* p = new DevPool();  // outlives every static DevArray
+BlockPool<HipMem>& pool() {
+  static auto* p = new BlockPool<HipMem>(kPoolBytes);  // outlives every static DevArray
   return *p;
 }
-// sizes that fit one another's blocks: steps of an eighth of the leading power of two
-size_t pool_round(size_t bytes) {
-  size_t step = 512;
-  while (step * 16 <= bytes) step <<= 1;
-  return (bytes + step - 1) / step * step;
+int alloc_failed(size_t bytes) {
+  set_error("hipMalloc of %zu bytes failed: %s", bytes, hipGetErrorString(g_alloc_err));
+  return -1;
 }
 }  // namespace
 
 int dev_alloc(void** p, size_t bytes, size_t* cap) {
-  DevPool& P = pool();
   int dev = 0;
   MH_HIP(hipGetDevice(&dev));
-  bytes = pool_round(bytes);
-  *cap = 0;
-  {
-    std::lock_guard<std::mutex> lk(P.mu);
-    if (P.device < 0) P.device = dev;
-    if (dev == P.device) {
-      *cap = bytes;
-      auto it = P.blocks.lower_bound(bytes);
-      if (it != P.blocks.end() && it->first <= bytes + bytes / 4) {
-        *p = it->second;
-        *cap = it->first;
-        P.cached -= it->first;
-        P.blocks.erase(it);
-        return 0;
-      }
-    }
-  }
-  if (hipMalloc(p, bytes) == hipSuccess) return 0;
-  (void)hipGetLastError();
-  std::multimap<size_t, void*> old;
-  {
-    std::lock_guard<std::mutex> lk(P.mu);
-    old.swap(P.blocks);
-    P.cached = 0;
-  }
-  for (auto& q : old) (void)hipFree(q.second);
-  MH_HIP(hipMalloc(p, bytes));
-  return 0;
+  return pool().alloc(p, bytes, dev, cap) ? 0 : alloc_failed(bytes);
 }
-
-// Called from destructors: nothing thrown leaves it.
-void dev_free(void* p, size_t cap) {
-  if (!p) return;
-  DevPool& P = pool();
-  bool kept = false;
-  if (cap > 0 && cap <= kPoolBytes) {
-    try {
-      std::lock_guard<std::mutex> lk(P.mu);
-      P.blocks.emplace(cap, p);
-      P.cached += cap;
-      kept = true;
-    } catch (...) {
-    }
-  }
-  if (!kept) (void)hipFree(p);
-  for (;;) {
-    void* q = nullptr;
-    {
-      std::lock_guard<std::mutex> lk(P.mu);
-      if (P.cached <= kPoolBytes) break;
-      auto it = std::prev(P.blocks.end());
-      P.cached -= it->first;
-      q = it->second;
-      P.blocks.erase(it);
-    }
-    (void)hipFree(q);
-  }
-}
+void dev_free(void* p, size_t cap) { pool().free(p, cap); }
+int dev_alloc_outside(void** p, size_t bytes) { return pool().alloc_outside(p, bytes) ? 0 : alloc_failed(bytes); }
+size_t dev_trim() { return pool().trim(); }
 
 template <typename T>
 int DevArray<T>::alloc(size_t count) {
