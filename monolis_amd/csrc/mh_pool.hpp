@@ -33,15 +33,16 @@ class BlockPool {
 
   // A block of at least `bytes` on device `dev` (the current one); *cap is handed
   // back to free.  A request that the memory does not hold beside the cached blocks
-  // gets them all freed.
+  // gets them all freed, and what fits exactly is not refused for its rounding.
   bool alloc(void** p, size_t bytes, int dev, size_t* cap) {
+    const size_t want = bytes;
     bytes = pool_round(bytes);
-    *cap = 0;
+    bool own = false;
     {
       std::lock_guard<std::mutex> lk(mu_);
       if (device_ < 0) device_ = dev;
-      if (dev == device_) {
-        *cap = bytes;
+      own = dev == device_ && bytes <= limit_;
+      if (own) {
         auto it = blocks_.lower_bound(bytes);
         if (it != blocks_.end() && it->first <= bytes + bytes / 4) {
           *p = it->second;
@@ -52,7 +53,10 @@ class BlockPool {
         }
       }
     }
-    return alloc_outside(p, bytes);
+    *cap = own ? bytes : 0;  // 0: freed at once
+    if (alloc_outside(p, own ? bytes : want)) return true;
+    *cap = 0;
+    return own && sys_.alloc(p, want);
   }
 
   // Called from destructors: nothing thrown leaves it.

@@ -99,6 +99,28 @@ def test_what_the_pool_holds_is_given_to_any_allocation_that_needs_it(tmp_path):
 """)
 
 
+def test_rounding_refuses_nothing_that_fits(tmp_path):
+    _run(tmp_path, r"""
+  M.left = 200 * GB;
+  BlockPool<Fake> P(4 * GB);
+  void *a, *b, *c;
+  size_t ca, cb, cc;
+  CHECK(P.alloc(&a, 196 * GB, 0, &ca) && M.left == 4 * GB);     // larger than any block kept: exactly its size
+  CHECK(P.alloc(&b, 3 * GB - 1, 0, &cb) && M.left == 1 * GB);   // rounded up
+  CHECK(P.alloc(&c, 1 * GB - 3, 0, &cc));
+  P.free(c, cc);
+  P.trim();
+  M.left -= 5;
+  CHECK(M.left == 1 * GB - 5);
+  CHECK(P.alloc(&c, 1 * GB - 6, 0, &cc));                       // its rounded size no longer fits
+  P.free(c, cc);
+  P.free(b, cb);
+  P.free(a, ca);
+  P.trim();
+  CHECK(M.live.empty() && M.left == 200 * GB - 5);
+""")
+
+
 def test_threads_share_the_pool(tmp_path):
     _run(tmp_path, r"""
   M.left = 1000 * GB;
