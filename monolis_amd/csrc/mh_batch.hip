@@ -857,8 +857,8 @@ int batch_create(Batch** out, int nsys, const int* sys_row_h, int n, int nz, con
   for (int k = 0; k < nsys; ++k)
     rs[k] = ResSystem{sys_slice[k], B->h_slices[k], sys_row_h[k], B->h_rows[k],
                       ((double)B->h_nnz[k] + 6.0 * B->h_rows[k]) * std::cbrt(std::max((double)B->h_rows[k], 1.0))};
-  MH_TRY(res_plan_build(B->res, rs, slice_ptr.data(), nslices, B->slice_ptr.p, B->col.p, B->rowlen.p, nullptr,
-                        cu_count_batch(), s));
+  res_plan_build(B->res, rs, slice_ptr.data(), nslices, B->slice_ptr.p, B->col.p, B->rowlen.p, nullptr,
+                 cu_count_batch(), s);
   if (B->res.fits) B->cfg = kCfgResident;
   MH_HIP(hipStreamSynchronize(s));
   *out = B.release();

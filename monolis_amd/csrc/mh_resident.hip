@@ -132,10 +132,16 @@ int occupancy(size_t lds, int* per_cu) {
 
 }  // namespace
 
-int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
-                   const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int cus,
-                   hipStream_t s) {
-  plan.fits = false;
+void ResPlan::clear() {
+  fits = false;
+  for (auto* d : {&mem, &expf, &lcol}) d->release();
+  for (auto* d : {&halo, &g_ptr, &ctl, &sticky}) d->release();
+  part.release();
+}
+
+static int build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
+                 const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int cus,
+                 hipStream_t s) {
   double W = 0.0;
   int maxrows = 1;
   for (const ResSystem& q : sys) {
@@ -249,6 +255,19 @@ int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* 
   plan.ticks_per_s = (double)khz * 1000.0;
   plan.fits = true;
   return 0;
+}
+
+void res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
+                    const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int cus,
+                    hipStream_t s) {
+  plan.fits = false;
+  if (!made_plan([&] {
+        return build(plan, sys, slice_ptr, nslices, d_slice_ptr, d_col, rowlen, rowptr, cus, s);
+      })) {
+    plan.fits = false;
+    clear_error();
+  }
+  if (!plan.fits) plan.clear();
 }
 
 int res_launch(const ResPlan& plan, const int* d_slice_ptr, const double* val, const double* dinv, const ResArgs& a,

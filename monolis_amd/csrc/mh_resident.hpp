@@ -525,14 +525,16 @@ struct ResPlan {
   DevArray<unsigned char> mem, expf, lcol;
   DevArray<int> halo, g_ptr, ctl, sticky;
   DevArray<unsigned long long> part;
+  void clear();  // no plan, no memory
 };
 
 // slice_ptr: host slot offsets of every slice; d_slice_ptr / d_col: the device
 // arrays (global 0-based columns); rowlen (per SELL row) or rowptr (per row)
 // gives the row lengths.  Plan.fits is false when a system needs more members than
 // a team may have or a member's rows and halo exceed LDS.  cus: the GPU's CUs, the
-// workgroups that the systems share.
-int res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
+// workgroups that the systems share.  A plan that does not fit, or that there is
+// no memory for, is cleared.
+void res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int* slice_ptr, int nslices,
                    const int* d_slice_ptr, const int* d_col, const int* rowlen, const int* rowptr, int cus,
                    hipStream_t s);
 // Zeroes the counters and enqueues the solver (both capturable).  A wait of a

@@ -2,8 +2,20 @@
 #pragma once
 
 #include <algorithm>
+#include <exception>
 
 namespace mh {
+
+// Whether build() made its plan: one that fails (memory) or throws is a system
+// that does not run on chip, not a failed call.
+template <class F>
+bool made_plan(F&& build) {
+  try {
+    return build() == 0;
+  } catch (const std::exception&) {
+    return false;
+  }
+}
 
 constexpr int kResNT = 512;                 // threads per member: two wavefronts per SIMD, 256 VGPRs each
 constexpr int kResNW = kResNT / 64;         // its wavefronts, one 64-row slice each at a time

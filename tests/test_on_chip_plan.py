@@ -29,11 +29,29 @@ int main() {
 """
 
 
-def test_members_of_a_team_fit_on_the_gpu_at_once(tmp_path):
+def _run(tmp_path, program):
     src, exe = tmp_path / "plan.cpp", tmp_path / "plan"
-    src.write_text(PROGRAM)
+    src.write_text(program)
     subprocess.run(["g++", "-O1", "-std=c++17", "-I", os.path.join(ROOT, "monolis_amd", "csrc"), str(src), "-o", str(exe)],
                    check=True)
     r = subprocess.run([str(exe)], capture_output=True, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
-    assert r.stdout.split() == ["64", "32", "3"], r.stdout
+    return r.stdout.split()
+
+
+def test_a_plan_without_memory_is_no_plan_and_no_error(tmp_path):
+    _run(tmp_path, r"""
+#include <new>
+#include <vector>
+#include "mh_resident_plan.hpp"
+int main() {
+  const bool ok = mh::made_plan([] { return 0; }) && !mh::made_plan([] { return -1; }) &&
+                  !mh::made_plan([]() -> int { throw std::bad_alloc(); }) &&
+                  !mh::made_plan([]() -> int { std::vector<int> v; return v.at(3); });
+  return ok ? 0 : 1;
+}
+""")
+
+
+def test_members_of_a_team_fit_on_the_gpu_at_once(tmp_path):
+    assert _run(tmp_path, PROGRAM) == ["64", "32", "3"]
