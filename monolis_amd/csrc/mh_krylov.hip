@@ -1296,18 +1296,27 @@ int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, doub
                SolveResult* out, bool* ran, hipStream_t s) {
   *ran = false;
   if (M.n < 1 || M.n != M.np || P.max_iter < 1 || P.steps || !M.on_chip || active_ktimer()) return 0;
-  if ((long long)M.nslices > (long long)kResTeamMax * kResRowsLarge * kResNW) return 0;
+  // With the matrix in registers always; otherwise while a member streams at
+  // most 300 KB per iteration (8 bytes of value and 2 of index per slot).  us per
+  // iteration in three launches / on chip, by KB per member: 13-point rows 48^3
+  // 112 KB 20.1 / 14.0, 27-point 40^3 138 KB 20.1 / 12.0, 48^3 233 KB 23.0 / 16.4,
+  // 57-point 40^3 292 KB 25.6 / 16.6.  The line is on the safe side: 27-point 64^3
+  // 553 KB 33.3 / 26.7, 76^3 926 KB 47.6 / 43.8, 125-point 48^3 1,080 KB 47.5 / 39.4,
+  // and lost with 125-point 12^3, one member of 2,160 KB, 32.2 / 44.8.
+  const int cus = cu_count(), T = res_members(M.nslices, cus, cus);
+  const bool streams_little = (double)M.nslots * kWave * 10.0 <= 300e3 * T;
+  const bool may_hold = M.max_width <= 8 && M.nslices <= T * kResRowsSmall * kResNW;
+  if (T == 0 || !(streams_little || may_hold)) return 0;
   if (!M.res) {
     M.res = new ResPlan();
     std::vector<int> sp((size_t)M.nslices + 1);
     MH_HIP(hipMemcpyAsync(sp.data(), M.slice_ptr.p, sizeof(int) * sp.size(), hipMemcpyDeviceToHost, s));
     MH_HIP(hipStreamSynchronize(s));
     res_plan_build(*M.res, {ResSystem{0, M.nslices, 0, M.n, 1.0}}, sp.data(), M.nslices, M.slice_ptr.p, M.col.p,
-                   nullptr, M.rowptr.p, cu_count(), s);
+                   nullptr, M.rowptr.p, cus, s);
+    if (!M.res->mr && !streams_little) M.res->clear();
   }
-  // With the matrix in registers always; otherwise while a member streams at
-  // most 300 KB per iteration (about 10 us from one CU).
-  if (!M.res->fits || (!M.res->mr && (double)M.nslots * kWave * 10.0 > 300e3 * M.res->nmem)) return 0;
+  if (!M.res->fits) return 0;
   struct Result {
     int iter, status;
     double resid;

@@ -2,6 +2,8 @@
 against the launch-per-step solver on the same handle (taken by a solve with the
 time split on) and the oracle: same status, iteration counts within +-2 % (+-1 below
 50), solutions within 1e-6."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -221,3 +223,60 @@ def test_on_chip_settings_reach_the_transpose():
     dm.set_on_chip(True)
     dm.solve_transpose(db, dx, _prm())
     assert dm.on_chip_solves() == (1, 1) and np.linalg.norm(dx.numpy() - xs) <= 1e-6 * np.linalg.norm(xs)
+
+
+def _matchings(n, count, seed):
+    """Rows of a diagonal and `count` random partners (symmetric): a member's rows couple to the whole system."""
+    rng = np.random.default_rng(seed)
+    i, j = [], []
+    for _ in range(count):
+        p = rng.permutation(n)[:n // 2 * 2].reshape(-1, 2)
+        i.append(p[:, 0])
+        j.append(p[:, 1])
+    i, j = np.concatenate(i), np.concatenate(j)
+    key = np.unique(np.concatenate([i * n + j, j * n + i, np.arange(n) * (n + 1)]))
+    rows, cols = key // n, key % n
+    index = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    return Matrix(n, n, 1, index, (cols + 1).astype(np.int32), np.where(rows == cols, count + 0.5, -1.0)).ensure_dof_index()
+
+
+# rows whose matrix is streamed and is too much for that (no plan is built); a halo that exceeds LDS (known
+# only once the plan is built)
+@pytest.mark.parametrize("make, built", [(lambda: _box27(56), False), (lambda: _matchings(400000, 7, 3), True)])
+def test_a_system_that_stays_off_the_chip_keeps_no_plan(hip, make, built):
+    def left():
+        free, total = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+        return free.value
+
+    mat = make()
+    b = W.uniform_vector(mat.n, seed=1)
+    dm = api.DeviceMatrix(mat)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
+    dm.set_on_chip(False)
+    dm.solve(db, dx, _prm())
+    x = dx.numpy()
+    api.trim()
+    before = left()
+    dm.set_on_chip(True)
+    for first in (True, False):
+        dm.solve(db, dx, _prm())
+        assert dm.on_chip_solves() == (0, 0) and np.array_equal(x, dx.numpy())
+        assert (api.trim() > 0) == (built and first) and left() == before
+
+
+def _box27(e):
+    n = e ** 3
+    ids = np.arange(n)
+    z, y, x = ids // (e * e), ids // e % e, ids % e
+    rows, cols = [], []
+    for dz in (-1, 0, 1):
+        for dy in (-1, 0, 1):
+            for dx in (-1, 0, 1):
+                ok = (z + dz >= 0) & (z + dz < e) & (y + dy >= 0) & (y + dy < e) & (x + dx >= 0) & (x + dx < e)
+                rows.append(ids[ok])
+                cols.append((ids + (dz * e + dy) * e + dx)[ok])
+    key = np.sort(np.concatenate(rows) * n + np.concatenate(cols))
+    rows, cols = key // n, key % n
+    index = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
+    return Matrix(n, n, 1, index, (cols + 1).astype(np.int32), np.where(rows == cols, 27.0, -1.0)).ensure_dof_index()
