@@ -86,7 +86,7 @@ struct ResArgs {
 struct ResShared {
   double red[2][2 * kResNW];
   double tot[2];
-  int ok, next, aborted;
+  int ok, next;
 };
 
 __device__ __forceinline__ void st_agent(double* p, double v) {
@@ -481,7 +481,8 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
 // members are consecutive, so at most one team is incomplete at any time and a
 // member waiting for a teammate that has not started waits only for running
 // workgroups to finish their own complete teams.  Members of teams that start
-// after a wait gave up report it at once.
+// after a wait gave up report it at once (the workgroup's first thread alone: a
+// branch around the solver's call raised its spilled registers from 8 to 37).
 template <int RP, bool MR>
 __global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP <= kResRowsSmall && !MR ? 4 : 2)))
     k_res_cg(ResView V, ResArgs a) {
@@ -489,17 +490,18 @@ __global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP 
   __shared__ ResShared sh;
   for (;;) {
     if (threadIdx.x == 0) {
-      sh.next = __hip_atomic_fetch_add(V.ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      sh.aborted = __hip_atomic_load(V.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      auto take = [&]() { return __hip_atomic_fetch_add(V.ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+      int k = take();
+      if (__hip_atomic_load(V.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
+        for (; k < V.nmem && V.mem[k].T > 1; k = take())
+          __hip_atomic_fetch_max(a.out.status + V.mem[k].sys, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      sh.next = k;
     }
     __syncthreads();
     const int k = __builtin_amdgcn_readfirstlane(sh.next);
     if (k >= V.nmem) break;
     const ResMember m = V.mem[k];
-    if (m.T > 1 && __builtin_amdgcn_readfirstlane(sh.aborted) != 0) {
-      if (threadIdx.x == 0)
-        __hip_atomic_fetch_max(a.out.status + m.sys, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    } else if constexpr (MR) {
+    if constexpr (MR) {
       res_cg<RP, true, true>(V, m, a, res_lds, sh);
     } else {
       if (m.w8) res_cg<RP, true, false>(V, m, a, res_lds, sh);
