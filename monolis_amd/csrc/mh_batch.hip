@@ -886,7 +886,7 @@ int batch_solve(Batch& B, const BatchParams& P, const double* b, double* x, int 
   if (grid < 1) grid = 1;
   auto enqueue = [&]() -> int {
     if (cfg == kCfgResident) {
-      const ResArgs A{b, x, z, p, q, O, nullptr, P.max_iter, P.tol, P.init_x, P.precond};
+      const ResArgs A{b, x, z, p, q, O, nullptr, nullptr, P.max_iter, P.tol, P.init_x, P.precond};
       return res_launch(B.res, B.slice_ptr.p, B.val.p, B.dinv.p, A, B.nsys, B.wait_s, s);
     }
     const int nctl = S ? 2 + S->nteam : 0;

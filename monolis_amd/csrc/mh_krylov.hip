@@ -1287,15 +1287,16 @@ size_t cg_bytes(const Matrix& M, int nvec, int max_iter) {
 // The on-chip CG on a scalar system (mh_resident.hpp): one launch instead of
 // three per iteration.  *ran stays false when the system does not fit, or when
 // a team's wait gave up (x is then as it was, and the matrix's later solves no
-// longer try); the launch-per-step solver follows.  Solves with a time split take
-// that one too: it times its steps.
+// longer try); the launch-per-step solver follows.  A time split is measured in
+// the kernel: products, update and preconditioner passes (one pass, as in the
+// launch-per-step solver) and the rest, vector updates and sums.
 // A team needs all of its workgroups (at most 128) on the GPU at once, which other
 // work on it can prevent: the wait limit is what that may cost a matrix, once
 // (0.5 s by default, against at most about 50 us between two exchanges).
 int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, double* x, Workspace& W,
                SolveResult* out, bool* ran, hipStream_t s) {
   *ran = false;
-  if (M.n < 1 || M.n != M.np || P.max_iter < 1 || P.steps || !M.on_chip || active_ktimer()) return 0;
+  if (M.n < 1 || M.n != M.np || P.max_iter < 1 || P.steps || !M.on_chip) return 0;
   // With the matrix in registers always; otherwise while a member streams at
   // most 300 KB per iteration (8 bytes of value and 2 of index per slot).  us per
   // iteration in three launches / on chip, by KB per member: 13-point rows 48^3
@@ -1320,7 +1321,8 @@ int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, doub
   struct Result {
     int iter, status;
     double resid;
-  } h{0, 3, 0.0};
+    long long ticks[3];
+  } h{0, 3, 0.0, {0, 0, 0}};
   const size_t m = (size_t)M.n;
   MH_TRY(W.ensure(4 * (m * sizeof(double) + 256) + ((size_t)P.max_iter + 2) * sizeof(double) + 1024));
   Carve cv{W.raw.p};
@@ -1331,9 +1333,10 @@ int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, doub
   double* hist = cv.take<double>((size_t)P.max_iter + 2);
   Result* d = cv.take<Result>(1);
   if (!P.init_x) MH_HIP(hipMemcpyAsync(x0, x, m * sizeof(double), hipMemcpyDeviceToDevice, s));
-  const ResArgs a{b, x, z, p, xe, {&d->iter, &d->resid, &d->status}, P.keep_hist ? hist : nullptr, P.max_iter, P.tol,
-                  P.init_x, prec ? 1 : 0};
+  const ResArgs a{b, x, z, p, xe, {&d->iter, &d->resid, &d->status}, P.keep_hist ? hist : nullptr,
+                  active_ktimer() ? d->ticks : nullptr, P.max_iter, P.tol, P.init_x, prec ? 1 : 0};
   MH_TRY(res_launch(*M.res, M.slice_ptr.p, M.val64.p, prec ? M.D64.p : nullptr, a, 1, M.on_chip_wait, s));
+  ktimer_mark(kClsDot);
   MH_HIP(hipMemcpyAsync(&h, d, sizeof(Result), hipMemcpyDeviceToHost, s));
   MH_HIP(hipStreamSynchronize(s));
   if (h.status < 0 || h.status > 2) {
@@ -1343,6 +1346,11 @@ int cg_on_chip(Matrix& M, const SolveParams& P, bool prec, const double* b, doub
     MH_TRY(res_aborted(*M.res, &gave_up, s));
     if (!P.init_x) MH_HIP(hipMemcpyAsync(x, x0, m * sizeof(double), hipMemcpyDeviceToDevice, s));
     return 0;
+  }
+  if (KTimer* t = active_ktimer()) {
+    const double ms = 1e3 / M.res->ticks_per_s;
+    t->move(kClsDot, kClsSpmv, ms * (double)h.ticks[0]);
+    t->move(kClsDot, prec ? kClsPrec : kClsDot, ms * (double)h.ticks[1]);
   }
   out->hist.clear();
   out->zero_rhs = h.status == 2;

@@ -87,6 +87,11 @@ struct KTimer {
     marks.push_back(Mark{e, cls});
     if (marks.size() > 256) harvest(false);
   }
+  // Charges t ms that one launch took for another class to that class.
+  void move(int from, int to, double t) {
+    ms[from] -= t;
+    ms[to] += t;
+  }
   // Charges every completed interval; with `wait` first waits for the last event.
   void harvest(bool wait) {
     if (wait && !marks.empty() && hipEventSynchronize(marks.back().ev) != hipSuccess) err = 1;

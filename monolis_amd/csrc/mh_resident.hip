@@ -1,6 +1,7 @@
 // Plans and launches of the on-chip CG (mh_resident.hpp).
 #include <algorithm>
 #include <cmath>
+#include <type_traits>
 #include <vector>
 
 #include "mh_resident.hpp"
@@ -122,9 +123,10 @@ constexpr size_t kResBuildLds = (size_t)120 << 10;
 // smaller plan would lower it below what an earlier one launches with).
 template <int RP, bool MR>
 int occupancy(size_t lds, int* per_cu) {
-  auto* k = &k_res_cg<RP, MR>;
-  MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k), hipFuncAttributeMaxDynamicSharedMemorySize,
-                             (int)(kResLds * sizeof(double))));
+  auto* k = &k_res_cg<RP, MR, false>;
+  for (auto* f : {k, &k_res_cg<RP, MR, true>})
+    MH_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(f), hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)(kResLds * sizeof(double))));
   *per_cu = 0;
   MH_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(per_cu, k, kResNT, lds));
   return 0;
@@ -280,10 +282,18 @@ int res_launch(const ResPlan& plan, const int* d_slice_ptr, const double* val, c
   const ResView V{plan.nmem, (const ResMember*)plan.mem.p, d_slice_ptr, plan.g_ptr.p, val, (const uint4*)plan.lcol.p,
                   plan.expf.p, dinv, plan.halo.p, plan.ctl.p, plan.part.p, (long long)(plan.ticks_per_s * wait_s),
                   plan.sticky.p};
-  if (plan.rp == kResRowsMini) k_res_cg<kResRowsMini, true><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
-  else if (plan.mr) k_res_cg<kResRowsSmall, true><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
-  else if (plan.rp == kResRowsSmall) k_res_cg<kResRowsSmall, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
-  else k_res_cg<kResRowsLarge, false><<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  auto launch = [&](auto rp, auto mr) {
+    auto* k = a.ticks ? &k_res_cg<decltype(rp)::value, decltype(mr)::value, true>
+                      : &k_res_cg<decltype(rp)::value, decltype(mr)::value, false>;
+    k<<<plan.grid, kResNT, plan.lds_bytes, s>>>(V, a);
+  };
+  using Mini = std::integral_constant<int, kResRowsMini>;
+  using Small = std::integral_constant<int, kResRowsSmall>;
+  using Large = std::integral_constant<int, kResRowsLarge>;
+  if (plan.rp == kResRowsMini) launch(Mini{}, std::true_type{});
+  else if (plan.mr) launch(Small{}, std::true_type{});
+  else if (plan.rp == kResRowsSmall) launch(Small{}, std::false_type{});
+  else launch(Large{}, std::false_type{});
   MH_HIP(hipGetLastError());
   return 0;
 }

@@ -77,6 +77,8 @@ struct ResArgs {
   double* xe;
   BatchOut out;
   double* hist;    // residual history of the only system, or null
+  long long* ticks;  // timed solves of one system: wall-clock ticks of the products, of the
+                     // update and preconditioner passes, and of the whole solve
   int max_iter;
   double tol;
   int init_x, precond;
@@ -118,8 +120,10 @@ __device__ __forceinline__ bool res_on(int left, int i) {
   return i * kResNW < left;
 }
 
-// One member's part of one system.
-template <int RP, bool W8, bool MR>
+// One member's part of one system.  TIMED: the first wavefront of the first member
+// also sums the time its products and its update and preconditioner passes take
+// (the same operations in the same order otherwise).
+template <int RP, bool W8, bool MR, bool TIMED>
 __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, const ResArgs& a, double* lds,
                                        ResShared& sh) {
   const int lane = threadIdx.x & (kWave - 1);
@@ -370,9 +374,24 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
       if (real) a.x[g] = zero ? 0.0 : xv(i, l);
     });
   };
+  long long t_start = 0, t_lap = 0, t_product = 0, t_update = 0;
+  // the time since the last call, after which q holds its results
+  auto lap = [&]() {
+#pragma unroll
+    for (int i = 0; i < RP; ++i) asm volatile("" : "+v"(q[i]));
+    const long long now = (long long)wall_clock64(), d = now - t_lap;
+    t_lap = now;
+    return d;
+  };
+  if constexpr (TIMED) t_start = (long long)wall_clock64();
   auto finish = [&](int iters, double resid, int st) {
     if (threadIdx.x == 0) {
       if (m.rank == 0) {
+        if constexpr (TIMED) {
+          a.ticks[0] = t_product;
+          a.ticks[1] = t_update;
+          a.ticks[2] = (long long)wall_clock64() - t_start;
+        }
         a.out.iters[m.sys] = iters;
         a.out.resid[m.sys] = resid;
       }
@@ -390,7 +409,9 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
   double B2 = 0.0, rho = 0.0, beta = 0.0, resid = 1.0;
   int it = 0;
   for (;;) {
+    if constexpr (TIMED) lap();
     product();
+    if constexpr (TIMED) t_product += lap();
     double rr = 0.0, rz = 0.0, none = 0.0;
     double alpha = 0.0;
     if (!resid_step) {
@@ -416,6 +437,7 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
       }
     }
     // r, then z = M^-1 r (kept in q's registers), (r, r), (r, z); z of exported slices goes out
+    if constexpr (TIMED) lap();
     for_rows([&](int i, int, bool real, int g) {
       double d;
       if constexpr (KEEP) d = dreg[i];
@@ -430,6 +452,7 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
       if ((exports >> i) & 1)
         if (real) st_agent(a.z + g, zv);
     });
+    if constexpr (TIMED) t_update += lap();
     if (resid_step) {
       __syncthreads();  // LDS reads of the product are done
       load_vec([&](int, int, int g) { return it > 0 ? ld_agent(a.p + g) : 0.0; }, it > 0 ? a.p : nullptr);
@@ -483,7 +506,7 @@ __device__ __forceinline__ void res_cg(const ResView& V, const ResMember& m, con
 // workgroups to finish their own complete teams.  Members of teams that start
 // after a wait gave up report it at once (the workgroup's first thread alone: a
 // branch around the solver's call raised its spilled registers from 8 to 37).
-template <int RP, bool MR>
+template <int RP, bool MR, bool TIMED>
 __global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP <= kResRowsSmall && !MR ? 4 : 2)))
     k_res_cg(ResView V, ResArgs a) {
   extern __shared__ double res_lds[];
@@ -502,10 +525,10 @@ __global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP 
     if (k >= V.nmem) break;
     const ResMember m = V.mem[k];
     if constexpr (MR) {
-      res_cg<RP, true, true>(V, m, a, res_lds, sh);
+      res_cg<RP, true, true, TIMED>(V, m, a, res_lds, sh);
     } else {
-      if (m.w8) res_cg<RP, true, false>(V, m, a, res_lds, sh);
-      else res_cg<RP, false, false>(V, m, a, res_lds, sh);
+      if (m.w8) res_cg<RP, true, false, TIMED>(V, m, a, res_lds, sh);
+      else res_cg<RP, false, false, TIMED>(V, m, a, res_lds, sh);
     }
     __syncthreads();
   }
@@ -541,6 +564,7 @@ void res_plan_build(ResPlan& plan, const std::vector<ResSystem>& sys, const int*
                    hipStream_t s);
 // Zeroes the counters and enqueues the solver (both capturable).  A wait of a
 // team's member for another lasts at most wait_s seconds; 0: teams give up at once.
+// With a.ticks the solve is timed.
 int res_launch(const ResPlan& plan, const int* d_slice_ptr, const double* val, const double* dinv, const ResArgs& a,
                int nsys, double wait_s, hipStream_t s);
 // 1 when a team wait gave up in any launch since the last call (synchronises).

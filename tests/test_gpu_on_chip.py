@@ -1,6 +1,6 @@
 """Scalar CG solves that run in one launch with the vectors on chip,
-against the launch-per-step solver on the same handle (taken by a solve with the
-time split on) and the oracle: same status, iteration counts within +-2 % (+-1 below
+against the launch-per-step solver on the same handle (`set_on_chip(False)`) and the
+oracle: same status, iteration counts within +-2 % (+-1 below
 50), solutions within 1e-6."""
 import ctypes
 
@@ -44,11 +44,10 @@ def _matrix(n, far, wide, seed):
     return Matrix(n, n, 1, index, (cols[order] + 1).astype(np.int32), vals[order]).ensure_dof_index()
 
 
-def _prm(precond=1, tol=1e-8, steps=False, init_x=True, max_iter=3000):
+def _prm(precond=1, tol=1e-8, init_x=True, max_iter=3000):
     prm = api.Prm().quiet()
     prm.Iarray[api.MONOLIS_PRM_I_PRECOND] = precond
     prm.Iarray[api.MONOLIS_PRM_I_MAX_ITER] = max_iter
-    prm.Iarray[api.MONOLIS_PRM_I_IS_MEASUREMENT] = int(steps)
     prm.Iarray[api.MONOLIS_PRM_I_IS_INIT_X] = int(init_x)
     prm.Rarray[api.MONOLIS_PRM_R_TOL] = tol
     return prm
@@ -66,10 +65,12 @@ def _both(mat, b, precond=1, x0=None, **kw):
     for steps in (False, True):
         if x0 is not None:
             dx.upload(x0)
-        prm = _prm(precond, steps=steps, init_x=x0 is None, **kw)
+        dm.set_on_chip(not steps)
+        prm = _prm(precond, init_x=x0 is None, **kw)
         h = dm.solve(db, dx, prm, hist_len=3001)
         it = int(prm.Iarray[api.MONOLIS_PRM_I_CUR_ITER])
         out.append((dx.numpy(), it, h, int(prm.Iarray[api.MONOLIS_PRM_I_IERR]), prm.Rarray[api.MONOLIS_PRM_R_CUR_RESID]))
+    assert dm.on_chip_solves() == (1, 0)
     (x, it, h, st, res), (xs, its, hs, sts, ress) = out
     assert st == sts and _near(it, its), (it, its)
     assert np.linalg.norm(x - xs) <= 1e-6 * np.linalg.norm(xs)
@@ -280,3 +281,34 @@ def _box27(e):
     rows, cols = key // n, key % n
     index = np.concatenate([[0], np.cumsum(np.bincount(rows, minlength=n))]).astype(np.int32)
     return Matrix(n, n, 1, index, (cols + 1).astype(np.int32), np.where(rows == cols, 27.0, -1.0)).ensure_dof_index()
+
+
+# one workgroup; teams with four and eight rows per thread and the matrix in registers; a streamed matrix;
+# 26 rows per thread
+@pytest.mark.parametrize("make", [lambda: _matrix(1000, 333, True, 1), lambda: W.poisson7(32), lambda: W.poisson7(72),
+                                  lambda: _box27(32), lambda: W.poisson7(78)])
+@pytest.mark.parametrize("precond", [1, 0])
+def test_time_output_does_not_change_the_solve(make, precond):
+    """The flags that ask for the time split (on by default) measure the same solve on chip: same bits of x and
+    of the history; the split's parts are positive and within the solution time, and 0 without the flags."""
+    mat = make()
+    b = W.uniform_vector(mat.n, seed=2)
+    dm = api.DeviceMatrix(mat)
+    db, dx = api.DeviceBuffer.from_numpy(b), api.DeviceBuffer(mat.n)
+    out = []
+    for k, flag in enumerate([None, api.MONOLIS_PRM_I_SHOW_TIME, api.MONOLIS_PRM_I_IS_MEASUREMENT,
+                              api.MONOLIS_PRM_I_SHOW_TIME_STATISTICS, None]):
+        prm = _prm(precond, max_iter=260)
+        if flag is not None:
+            prm.Iarray[flag] = 1
+        h = dm.solve(db, dx, prm, hist_len=261)
+        assert dm.on_chip_solves() == (k + 1, 0)
+        out.append((dx.numpy(), h, int(prm.Iarray[api.MONOLIS_PRM_I_CUR_ITER])))
+        total, spmv, dotp, prec, c0, c1 = prm.Rarray[[3, 5, 6, 7, 8, 9]]
+        assert c0 == c1 == 0
+        if flag is None:
+            assert spmv == dotp == prec == 0
+        else:
+            assert spmv > 0 and dotp > 0 and (prec > 0) == bool(precond) and spmv + dotp + prec <= total
+    for x, h, it in out[1:]:
+        assert np.array_equal(x, out[0][0]) and np.array_equal(h, out[0][1]) and it == out[0][2]
