@@ -748,6 +748,21 @@ bool elem_rows_fit(const Matrix& M, int n_base) {
          (long long)n_base * M.b * M.b < (1LL << 30);
 }
 
+// Whether a call of n_elem elements is worth a pass over every block row: the pass
+// and the adjacency cost the same however few rows the elements touch.  us of a
+// call by rows / by sorted pairs, device inputs, consecutive hexahedra, 3 DOF:
+// 4,913 nodes: 64 elements 98 / 85, 1,024 135 / 122, 2,048 123 / 149, 4,096 145 /
+// 209; 274,625 nodes: 64 147 / 85, 2,048 171 / 149, 4,096 194 / 212, 65,536 389 /
+// 1,334 (scattered elements: 4,096 314 / 223, 16,384 489 / 554): a node pair per
+// block row, and 2^16 of them.  Rows too long for 16 of them in a workgroup's LDS
+// cost more to pass over (20-node elements, 3 DOF, 274,625 nodes: 64 elements 429
+// / 127, 4,096 592 / 615, scattered 1,653 / 742, 16,384 866 / 2,200): eight pairs.
+template <typename V>
+bool elem_rows_pay(const Matrix& M, long long pairs) {
+  const bool short_rows = (size_t)16 * M.max_width * M.b * M.b * sizeof(V) <= kElemLds;
+  return pairs >= std::max(1LL << 16, (long long)M.n * (short_rows ? 1 : 8));
+}
+
 template <typename V>
 int launch_elem_rows(const Matrix& M, int n_base, const Adjacency& adj, const unsigned short* pos, const V* Ke, V* val,
                      hipStream_t s) {
@@ -883,9 +898,9 @@ static int add_elements_T(Matrix* M, int n_elem, int n_base, const int* elem, co
     set_error("element connectivity holds a node id outside 0..%d", M->n - 1);
     return -2;
   }
-  // By block row when no element lists a node twice and four rows fit in a
-  // workgroup's LDS; otherwise by sorted node pairs.
-  const bool by_rows = !chk[1] && elem_rows_fit<V>(*M, n_base);
+  // By block row when no element lists a node twice, four rows fit in a
+  // workgroup's LDS and the elements are enough; otherwise by sorted node pairs.
+  const bool by_rows = !chk[1] && elem_rows_fit<V>(*M, n_base) && elem_rows_pay<V>(*M, n_elem * pairs_elem);
   int bad = 0;
   const bool ke_dev = is_device_pointer(Ke);
   const long long cap = (long long)chunk * pairs_elem;

@@ -86,6 +86,45 @@ def test_element_assembly_layouts_bit_identical(n_base, b, n_node, n_elem, dup):
     assert np.array_equal(dm.values(), mo.A)
 
 
+# both sides of the rule between block rows and sorted pairs (2^16 node pairs, one or eight per block row):
+# strips of one, two, four and more 64-value pieces; 16, 8 and 4 rows of LDS per workgroup; rows without an
+# element between rows with many
+ROWS_OR_PAIRS = [(8, 3, 500, 1023), (8, 3, 500, 1024), (2, 4, 700, 16384), (1, 1, 70001, 70001), (4, 1, 70001, 4200),
+                 (4, 1, 70001, 4400), (4, 5, 200, 4100), (10, 6, 90, 660), (20, 2, 150, 170), (8, 8, 130, 1030),
+                 (8, 8, 9000, 1050), (8, 8, 9000, 1200)]
+
+
+@pytest.mark.parametrize("n_base, b, n_node, n_elem, cplx",
+                         [(*c, False) for c in ROWS_OR_PAIRS] +
+                         [(*c, True) for c in ROWS_OR_PAIRS if c[:2] in ((8, 3), (2, 4), (10, 6), (4, 1))])
+def test_element_assembly_by_rows_and_by_pairs_bit_identical(n_base, b, n_node, n_elem, cplx):
+    rng = np.random.default_rng(n_base * 100 + b)
+    used = max(n_base, n_node * 3 // 4)
+    elems = (np.arange(n_elem)[:, None] * 7 + np.cumsum(rng.integers(1, 3, (n_elem, n_base)), 1)) % used
+    elems = elems.astype(np.int32)
+    create = api.device_matrix_by_simple_mesh_C if cplx else api.device_matrix_by_simple_mesh
+    dm = create(n_node, b, elems)
+    Ke = element_matrices(n_elem, n_base * b, seed=b, spd=False)
+    parts = [Ke, element_matrices(n_elem, n_base * b, seed=b + 1, spd=False)] if cplx else [Ke]
+    want = []
+    start = rng.uniform(-1, 1, (2, len(dm.mat.item) * b * b))
+    for k, K in enumerate(parts):
+        mo = _oracle_mat(n_node, b, elems)
+        assert np.array_equal(dm.mat.index, mo.index) and np.array_equal(dm.mat.item, mo.item)
+        mo.A[:] = start[k]
+        oracle.add_elements(mo, elems, K)
+        want.append(mo.A.copy())
+    if cplx:
+        dm.set_values(start[0] + 1j * start[1])
+        dm.add_elements(elems, parts[0] + 1j * parts[1])
+        v = dm.values()
+        assert np.array_equal(v.real, want[0]) and np.array_equal(v.imag, want[1])
+    else:
+        dm.set_values(start[0])
+        dm.add_elements(elems, Ke)
+        assert np.array_equal(dm.values(), want[0])
+
+
 def test_pattern_rejects_bad_node_ids():
     h = ctypes.c_void_p()
     e = np.array([[0, 5]], np.int32)
