@@ -34,7 +34,8 @@ struct RhsState {
 
 struct MState {
   int all_done;
-  int pad[63];
+  int last;  // the last iteration that ran
+  int pad[62];
 };
 
 // Lane layout: kk = 2^ks >= k lanes per row, 64/kk rows per wavefront step;
@@ -409,12 +410,15 @@ __device__ __forceinline__ void st_vec(T* p, T v) {
 // and q then move 7.5 times instead of 9 (the update reads q, r and writes r; the
 // p steps read r, p and write p, every second one also p and x twice).  96^3 x 64
 // right-hand sides: 776 -> 646 us per iteration for the two passes, 5.3 TB/s.
-// `pa`, `pb`: the p buffers of iterations it - 1 and it (MODE 0, 4); `it0` > 0: the
+// `pa`, `pb`: the p buffers of iterations it - 1 and it (MODE 0, 4); it = it0 > 0: the
 // iteration of p in the buffer it0 & 1 (MODE 2).
 //   MODE 0: p = z + beta p
 //   MODE 4: x += the multiples of p of iterations it - 2 and it - 1; p = z + beta p
 //   MODE 1: r -= alpha q; partial (r, r), (r, z)
-//   MODE 2: x += the multiples of p of iterations it0 and it0 + 1 that were run
+//   MODE 2: x += the multiples of p of iterations it0 and it0 + 1 that were run;
+//           it0 < 0: after the last iteration, of those that x still lacks (it lacks
+//           them from the last odd iteration on, unless that is past a residual
+//           replacement, which applies them first)
 //   MODE 3: partial (r, r), (r, z)
 // A right-hand side that is done keeps its r and p; its last one or two multiples
 // are applied by the next MODE 4 or 2 pass, which takes only the iterations it ran.
@@ -424,7 +428,13 @@ __global__ void __launch_bounds__(kBlock) k_mrows(int n, int k, int ks, T* __res
                                                   const T* __restrict__ q, const T* __restrict__ dinv,
                                                   double* __restrict__ partials, const MState* ms,
                                                   const RhsState* __restrict__ rs, int it) {
-  if (ms && ms->all_done) return;  // (null: the pass after the last iteration)
+  if (MODE == 2 && it < 0) {
+    const int last = ms->last;
+    if (last % kIterRR == 0) return;
+    it = last - (last % 2 == 0 ? 1 : 0);
+  } else if (ms->all_done) {
+    return;
+  }
   const Lanes L(k, ks);
   const int w = threadIdx.x / kWave;
   bool active = false;
@@ -614,13 +624,16 @@ __global__ void __launch_bounds__(kFinal) k_mfinal(int k, int ntiles, const doub
     done = st.done;
   }
   const bool all = __all(done);
-  if (j == 0) ms->all_done = all ? 1 : 0;
+  if (j == 0) {
+    ms->all_done = all ? 1 : 0;
+    if (STAGE == 1 && check) ms->last = it;
+  }
 }
 
 __global__ void k_mstate_init(int k, MState* ms, RhsState* rs) {
   const int j = threadIdx.x;
   if (j < k) rs[j] = RhsState{};
-  if (j == 0) ms->all_done = 0;
+  if (j == 0) ms->all_done = ms->last = 0;
 }
 
 template <typename T>
@@ -837,25 +850,23 @@ int multi_cg(Matrix& M, const MultiParams& P, int k, const T* b, T* x, Workspace
 
   k_mstate_init<<<1, kWave, 0, s>>>(k, ms, rs);
   if (P.init_x) k_mfill<T><<<grid_for(npk), kBlock, 0, s>>>(npk, x);
-  for (T* p : P2) k_mfill<T><<<grid_for(npk), kBlock, 0, s>>>(npk, p);
+  const size_t np2 = (off_q - off_p) / sizeof(T);  // both p buffers
+  k_mfill<T><<<grid_for(np2), kBlock, 0, s>>>(np2, P2[0]);
   // R = B - A X, B2 = (R, R)
   spmm<T, 2>(M, k, ks, cfg, val, x, b, r, parts, nullptr, sp_tiles, s);
   k_mfinal<0><<<1, kFinal, 0, s>>>(k, sp_tiles, parts, ms, rs, 0, 0, 0, P.tol, P.max_iter);
   // Z = M^-1 R, rho = (R, Z)
-  auto rows = [&](auto mode, int i, bool end = false) {
+  auto rows = [&](auto mode, int i) {
     constexpr int MODE = decltype(mode)::value;
-    // MODE 2: iteration i's p in the pp role (pb), iteration i + 1's in pa
-    const T* pa = MODE == 2 ? P2[(i + 1) & 1] : P2[(i - 1) & 1];
-    k_mrows<T, MODE><<<rw_tiles, kBlock, 0, s>>>(n, k, ks, x, r, pa, P2[i & 1], q, dinv, parts, end ? nullptr : ms, rs, i);
+    // MODE 2: the p of the first, odd iteration in the pp role (pb), the second's in pa
+    const int b2 = MODE == 2 ? 1 : i & 1;
+    k_mrows<T, MODE><<<rw_tiles, kBlock, 0, s>>>(n, k, ks, x, r, P2[b2 ^ 1], P2[b2], q, dinv, parts, ms, rs, i);
   };
   using M0 = std::integral_constant<int, 0>;
   using M1 = std::integral_constant<int, 1>;
   using M2 = std::integral_constant<int, 2>;
   using M3 = std::integral_constant<int, 3>;
   using M4 = std::integral_constant<int, 4>;
-  // x lacks the multiples of iterations from the last odd one on, unless that is
-  // past a residual replacement (which applies them first)
-  auto x_pending = [&](int last) { return last % kIterRR == 0 ? 0 : last - (last % 2 == 0 ? 1 : 0); };
   rows(M3{}, 0);
   k_mfinal<1><<<1, kFinal, 0, s>>>(k, rw_tiles, parts, ms, rs, 0, 0, 1, P.tol, P.max_iter);
   MH_HIP(hipGetLastError());
@@ -883,6 +894,8 @@ int multi_cg(Matrix& M, const MultiParams& P, int k, const T* b, T* x, Workspace
     MH_HIP(hipStreamSynchronize(s));
     if (*hflag) break;
   }
+  rows(M2{}, -1);
+  MH_HIP(hipGetLastError());
   std::vector<RhsState> hs(k);
   MH_HIP(hipMemcpyAsync(hs.data(), rs, sizeof(RhsState) * k, hipMemcpyDeviceToHost, s));
   MH_HIP(hipStreamSynchronize(s));
@@ -893,11 +906,6 @@ int multi_cg(Matrix& M, const MultiParams& P, int k, const T* b, T* x, Workspace
     out->resid[j] = hs[j].resid;
     out->status[j] = hs[j].zero ? 2 : (hs[j].conv ? 0 : 1);
     out->loop_iters = std::max(out->loop_iters, out->iters[j]);
-  }
-  if (const int i0 = out->loop_iters > 0 ? x_pending(out->loop_iters) : 0) {
-    rows(M2{}, i0, true);
-    MH_HIP(hipGetLastError());
-    MH_HIP(hipStreamSynchronize(s));
   }
   if (zero_mask) {
     k_zero_cols<T><<<grid_for(nk), kBlock, 0, s>>>(nk, k, zero_mask, x);
