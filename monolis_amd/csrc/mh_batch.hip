@@ -739,7 +739,7 @@ int batch_schedule_info(Batch& B, int cfg, int* split, int* nslot, int* nteam, h
 int batch_aborted(Batch& B, int cfg, int* aborted, hipStream_t s) {
   *aborted = 0;
   cfg = effective_config(B, cfg);
-  if (cfg == kCfgResident) return res_aborted(B.res, aborted, s);
+  if (cfg == kCfgResident) return B.res.nteam > 0 ? res_aborted(B.res, aborted, s) : 0;  // without teams nobody waits
   if (cfg < 0 || cfg >= (int)B.sched.size() || !B.sched[cfg] || batch_config_split(cfg) == 0) return 0;
   // the sticky flag: set by any launch since the last check, then cleared
   int flag = 0;
