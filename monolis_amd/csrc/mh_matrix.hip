@@ -188,6 +188,7 @@ int upload(void* dst, const void* src, size_t bytes, hipStream_t s) {
 
 int Workspace::ensure(size_t need) {
   if (need <= bytes) return 0;
+  bytes = 0;  // the old block is gone also when the new one cannot be had
   MH_TRY(raw.alloc(need));
   bytes = need;
   return 0;
