@@ -6,9 +6,9 @@
 //   * batched element matrices (monolis_add_matrix_to_sparse_matrix_main_R,
 //     src/matrix/spmat_handler_util.f90:398-497): the node pairs of all
 //     elements grouped by block row (by block position for elements that list a
-//     node twice or very long rows) in element order, then every block component
-//     summed left to right onto its current value, so the result equals one
-//     add-matrix call per element in element order, bit for bit;
+//     node twice, very long rows or few elements) in element order, then every block
+//     component summed left to right onto its current value, so the result equals
+//     one add-matrix call per element in element order, bit for bit;
 //   * Dirichlet conditions (monolis_set_Dirichlet_bc_main_R,
 //     src/matrix/spmat_handler_util.f90:604-677) for a whole list in one pass;
 //   * value and pattern read-back in monolis's layout.

@@ -12,9 +12,9 @@ namespace mh {
 // the reciprocal pivots.  With DOT, also the partial (src, dst) and, in
 // finalize, CG's rho = (r, z) and beta = rho / rho_prev (0 when `first`),
 // CG.f90:71-84, or with `first` = 2 GropCG's gamma = (r, u).
-// Block rows go in 256-thread workgroups (kVPrecBS sets the row kernels' size;
-// the op does its own loads): 85,184 block rows in 1024-thread ones reached 84 of
-// 256 CUs.  Blocks of up to kVPrecRegs rows run with every factor loaded up front
+// FP64 block rows go in 256-thread workgroups (kVPrecBS sets the row kernels' size
+// by the bytes of that many values; the op does its own loads): 85,184 block rows
+// in 1024-thread ones, which FP32 keeps, reached 84 of 256 CUs.  Blocks of up to kVPrecRegs rows run with every factor loaded up front
 // into registers; as loops over the block's size the working vector was indexed
 // dynamically, in scratch memory, and each factor waited for (24.8 -> 7.3 us with
 // blocks of 1, 2, 3 and 6; both orders of arithmetic are the same).

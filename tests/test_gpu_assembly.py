@@ -62,8 +62,8 @@ def test_pattern_hub_node_takes_the_sorted_pairs():
     assert np.array_equal(dm.mat.index, index) and np.array_equal(dm.mat.item, item)
 
 
-# strips of one, two, four and more 64-value pieces; 16, 8 and 4 rows of LDS per workgroup; rows too
-# long for LDS; an element that lists a node twice
+# few elements, which are summed by sorted pairs, in blocks of 1 to 8, one that lists a node twice (the same
+# layouts by block row: test_element_assembly_by_rows_and_by_pairs_bit_identical)
 @pytest.mark.parametrize("n_base, b, n_node, n_elem, dup",
                          [(1, 1, 5, 9, False), (2, 4, 67, 150, False), (8, 1, 300, 700, False), (4, 5, 200, 500, False),
                           (10, 6, 90, 130, False), (20, 2, 150, 100, False), (8, 8, 130, 260, False),
