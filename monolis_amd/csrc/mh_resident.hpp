@@ -514,8 +514,10 @@ __global__ void __launch_bounds__(kResNT) __attribute__((amdgpu_waves_per_eu(RP 
   for (;;) {
     if (threadIdx.x == 0) {
       auto take = [&]() { return __hip_atomic_fetch_add(V.ctl, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+      // both on their way at once
+      const int aborted = __hip_atomic_load(V.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       int k = take();
-      if (__hip_atomic_load(V.ctl + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0)
+      if (aborted != 0)
         for (; k < V.nmem && V.mem[k].T > 1; k = take())
           __hip_atomic_fetch_max(a.out.status + V.mem[k].sys, 3, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       sh.next = k;
